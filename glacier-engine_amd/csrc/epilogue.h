@@ -49,13 +49,35 @@ static __device__ __forceinline__ ArgPartial arg_shfl_xor(const ArgPartial &p, i
   return q;
 }
 
+// Power-of-two scale of a split-16 group: y = v * inv has max |y| in
+// [2^14, 2^15); `scale` = 2^10 / inv undoes half_codes' factor as well, so
+// scale times the dot of y with the half codes is the dot of v with u - 7.
+// Values under 2^-112 share the smallest scale.
+static __device__ __forceinline__ float split16_scale(float amax, float *scale) {
+  const uint32_t e = max(__float_as_uint(amax) >> 23, 15u);
+  *scale = __uint_as_float((e - 14u + 10u) << 23);
+  return __uint_as_float((268u - e) << 23);
+}
+
 // Converts the 32-element group held by a 32-lane half-wave (one value per
-// lane, hl = lane within the half-wave) into D digit bytes per lane and the
-// group's meta. q layout [G][D][M][32], meta [G][M].
+// lane, hl = lane within the half-wave) into planes of layout D (kernels.h)
+// and the group's meta.
 template <int D>
 static __device__ __forceinline__ void quantize_group(float v, int hl, int g, int m, int M,
                                                       int8_t *act_q, ActMeta *meta) {
   const float amax = half_wave_max(fabsf(v));
+  if constexpr (D == kPlanesSplit16) {
+    ActMeta mm;
+    const float y = v * split16_scale(amax, &mm.scale);
+    const _Float16 hi = (_Float16)y;
+    const _Float16 lo = (_Float16)(y - (float)hi);
+    _Float16 *q = (_Float16 *)act_q;
+    q[(((size_t)g * 2 + 0) * M + m) * 32 + split16_pos(hl)] = hi;
+    q[(((size_t)g * 2 + 1) * M + m) * 32 + split16_pos(hl)] = lo;
+    mm.corr = 0;
+    if (hl == 0) meta[(size_t)g * M + m] = mm;
+    return;
+  }
   const float scale = amax / 127.0f;
   const float inv_s = scale == 0.0f ? 0.0f : 1.0f / scale;
   const float y = v * inv_s;
@@ -82,6 +104,14 @@ static __device__ __forceinline__ void quantize_group(float v, int hl, int g, in
     mm.corr = 7 * sum;
     meta[(size_t)g * M + m] = mm;
   }
+}
+
+// The same for a layout chosen at run time.
+static __device__ __forceinline__ void quantize_group_d(int D, float v, int hl, int g, int m,
+                                                        int M, int8_t *act_q, ActMeta *meta) {
+  if (D == kPlanesQ8) quantize_group<kPlanesQ8>(v, hl, g, m, M, act_q, meta);
+  else if (D == kPlanesSplit16) quantize_group<kPlanesSplit16>(v, hl, g, m, M, act_q, meta);
+  else quantize_group<kPlanesDigits>(v, hl, g, m, M, act_q, meta);
 }
 
 static __device__ __forceinline__ float silu_mul(float g, float u) {

@@ -1,40 +1,37 @@
-// gemm.hip — K2: INT4 x int8-digit GEMM on gfx950 MFMA.
+// gemm.hip — K2: INT4 x activation-plane GEMM on gfx950 MFMA.
 //
-// y[M][N] = planes(x)[M][K] . W^T past the decode GEMV's rows (decode
-// batches of 6 or more lanes, prompt chunks), with the
-// same digit planes, tile layout and fused epilogues as the decode GEMV (K1):
-// the per-group arithmetic is the reference's Q8 dot
-// (int4_matmul.zig:365-418): an exact integer dot per 32-element group,
-// scaled by the weight and activation group scales and summed in f32.
+// y[M][N] = planes(x)[M][K] . W^T past the decode GEMV's rows (decode batches
+// of 3 or more lanes, prompt chunks), with the same tile layout and fused
+// epilogues as the decode GEMV (K1). Two plane layouts (kernels.h):
+//   * Q8: the per-group arithmetic is the reference's Q8 dot
+//     (int4_matmul.zig:365-418), an exact integer dot per 32-element group
+//     scaled by the weight and activation group scales and summed in f32. One
+//     i8 MFMA with K = 32 covers one group of an output tile. The codes are
+//     made signed (u - 7), so its result is the group dot T itself; the
+//     accumulator starts at the bits of 1.5 * 2^23 and fma(that as f32, ws,
+//     -12582912 * ws) = RN(T * ws) (int4_ops.h), then one fma applies the
+//     activation scale into the running sum.
+//   * split-16: f32 activations as an fp16 pair per element (x / 2^e = hi + lo
+//     to 2^-23 of x), codes as exact halves, two fp16 MFMAs (one onto the
+//     other) per group with f32 accumulation, then the same two scales. Against
+//     three 7-bit digits on i8 MFMAs (three of them and five f32 / integer
+//     operations per output and group): 1999 x 3584 x 18944 1298 -> 845 us,
+//     error against 64-bit sums 5.9e-7 -> 1.8e-7.
 //
-// One v_mfma_i32_16x16x32_i8 covers exactly one group of a 16x16 output tile.
-// The weight codes are made signed (u - 7) in registers, so the MFMA result
-// is the group dot T itself; with one digit the accumulator starts at the
-// bits of 1.5 * 2^23 and fma(that as f32, ws, -12582912 * ws) = RN(T * ws)
-// (int4_ops.h), then one fma applies the activation scale into the running
-// sum. Three-digit (f32 activation) planes run three independent MFMAs and
-// combine them as the exact 128-adic integer.
-//
-// The per-group scaling (two fmas per output and group against one MFMA per
-// 16 x 16 x 32 group tile) bounds this kernel by VALU issue, not by the
-// matrix cores; the layout keeps everything else off that path:
-//   * workgroup = 4 waves over a BM-row (32 or 64) x 64 kRB-column output
-//     tile; each wave owns kRB (1, 2 or 4) weight row blocks x the BM / 16
-//     activation row tiles;
-//   * weights: each lane loads its own 16-byte tile slot per row block and
-//     quad (1 KB per wave, fully coalesced), two quads in flight; the words
-//     are transposed across lanes into MFMA operands (quad_transpose) and
-//     the lane-ordered fp16 scales gathered per column (column_gather);
-//   * activations: the workgroup stages each quad's digit planes (64 rows x
-//     128 columns x D) and their scales in LDS, double buffered, one barrier
-//     per quad; every wave reads its operands from there;
-//   * block ids are remapped so that the row tiles of one weight column tile
-//     run on one XCD (hardware places block b on XCD b % 8), which keeps the
-//     tile's weights in that XCD's L2 for every row tile that reads them;
-//   * small grids (few row tiles x few column tiles, e.g. 32 decode rows of a
-//     3584-wide projection) split K over workgroups: each split writes its
-//     partial sums and splitk_reduce_kernel adds the splits in a fixed order
-//     and runs the epilogue (deterministic, no atomics).
+// The per-group scaling (two f32 operations per output and group) bounds the
+// tall tiles by vector issue, not by the matrix cores. Two kernels:
+//   * up to 32 rows, gemm_kernel: 4 waves over 16 or 32 rows, each wave its
+//     own weight row blocks. Each lane loads its own 16-byte tile slot per row
+//     block and quad (1 KB per wave, fully coalesced), two quads in flight;
+//     the words are transposed across lanes into MFMA operands
+//     (quad_transpose) and the lane-ordered fp16 scales gathered per column
+//     (column_gather). The workgroup stages each quad's activation planes in
+//     LDS, double buffered, one barrier per quad;
+//   * prompt chunks, gemm_tile_kernel: 64 or 128 rows x 128 columns by 8
+//     waves, both operands in LDS.
+// Small grids split K over workgroups: each split writes its partial sums and
+// a finishing kernel (or the last split to arrive) adds them in a fixed order
+// and runs the epilogue (deterministic).
 #include "epilogue.h"
 #include "int4_ops.h"
 #include "kernels.h"
@@ -45,91 +42,124 @@ namespace gk {
 
 namespace {
 
+typedef float v4f __attribute__((ext_vector_type(4)));
+typedef int v16i __attribute__((ext_vector_type(16)));
+typedef long v2l __attribute__((ext_vector_type(2)));
+
 constexpr int kWaves = 4;            // waves per workgroup, side by side in N
 constexpr int kU = 2;                // weight quads in flight per wave
 constexpr int kFoldSplits = 4;       // K splits a folded tile adds at most
 
-// Per-quad activation staging of a BM-row tile: digit planes
-// [4 groups][D][BM rows][32] then the scales [4][BM].
+// Activation staging of the 16- and 32-row tiles: a quad's planes as 16-byte
+// units, then the group scales [4][BM].
+//   Q8:       [group][half][row][16 B], a half's stride padded by 64 bytes;
+//   split-16: [group][hi, lo][unit][row][16 B], a unit's stride padded by 32.
+// A wave's operand read takes 16 bytes of consecutive rows (no bank
+// conflicts), and the pads keep the staging writes, whose lanes take the
+// units of a row in turn, on distinct banks.
 template <int D, int BM>
 struct ActStage {
-  static constexpr int kActBytes = 4 * D * BM * 32;
-  static constexpr int kBufBytes = kActBytes + 4 * BM * 4;
-  static constexpr int kUnitCount = kActBytes / 16;            // 16-byte units
-  static constexpr int kUnits = (kUnitCount + 255) / 256;      // per thread
+  static constexpr int SG = 4;
+  static constexpr int kRowUnits = D == kPlanesQ8 ? 2 : 4;      // per plane row
+  static constexpr int kPlanes = D == kPlanesQ8 ? 1 : 2;        // planes per group
+  static constexpr int kUnitStride = BM * 16 + (D == kPlanesQ8 ? 64 : 32);
+  static constexpr int kPlaneStride = kRowUnits * kUnitStride;
+  static constexpr int kActBytes = SG * kPlanes * kPlaneStride;
+  static constexpr int kBufBytes = kActBytes + SG * BM * 4;
+  static constexpr int kUnitCount = SG * kPlanes * BM * kRowUnits;
+  static constexpr int kUnits = (kUnitCount + 255) / 256;       // per thread
+  static_assert(kUnits <= 4 && SG * BM <= 256, "ActRegs holds four units and a scale per thread");
 };
 
-// One thread's share of a quad's activation staging: up to six 16-byte
-// units (3-digit planes, 64 rows) as named members, read and written through
-// at() with indices that are constants once the loops are unrolled. (An
-// array member of six units was kept in scratch memory, whose stores waited
-// for the loads as soon as they were issued.)
-template <int D, int BM>
+// One thread's share of a stage as named members, read and written through
+// at() with indices that are constants once the loops are unrolled (an array
+// member of them was kept in scratch memory, whose stores waited for the
+// loads as soon as they were issued).
 struct ActRegs {
-  static_assert(ActStage<D, BM>::kUnits <= 6, "six units per thread at most");
-  uint4 v0, v1, v2, v3, v4, v5;
+  uint4 v0, v1, v2, v3;
   float sc;
   __device__ __forceinline__ uint4 &at(int i) {
     switch (i) {
       case 0: return v0;
       case 1: return v1;
       case 2: return v2;
-      case 3: return v3;
-      case 4: return v4;
-      default: return v5;
+      default: return v3;
     }
-  }
-  __device__ __forceinline__ const uint4 &at(int i) const {
-    return const_cast<ActRegs *>(this)->at(i);
   }
 };
 
-// Loads quad kq's activation planes (rows m0 .. m0 + BM - 1, clamped to
-// M - 1) and scales into registers; one 16-byte unit per thread and pass
-// (16-row tiles have fewer units than threads: the extra threads repeat the
-// last unit, branch-free).
+// Where a thread's units and scale of a stage lie: byte offsets from the
+// stage's first group in the planes (rows m0 .. m0 + BM - 1, clamped to
+// M - 1) and into the LDS buffer. Loads are base + 32-bit offset.
 template <int D, int BM>
-__device__ __forceinline__ ActRegs<D, BM> act_load(const GemvArgs &p, int kq, int m0) {
-  ActRegs<D, BM> r;
-  const int M = p.M, t = threadIdx.x;
+struct ActMap {
+  using S = ActStage<D, BM>;
+  uint32_t src[S::kUnits], dst[S::kUnits], msrc, mdst;
+  __device__ __forceinline__ ActMap(int M, int m0) {
+    const int t = threadIdx.x;
 #pragma unroll
-  for (int i = 0; i < ActStage<D, BM>::kUnits; ++i) {
-    const int u = min(t + 256 * i, ActStage<D, BM>::kUnitCount - 1);  // ((j * D + d) * BM + row) * 2 + half
-    const int half = u & 1, row = (u >> 1) % BM, jd = (u >> 1) / BM;
-    const int m = min(m0 + row, M - 1);
-    const size_t src = ((size_t)(4 * kq) * D + jd) * M + m;  // group 4kq + j, digit d
-    r.at(i) = *(const uint4 *)(p.act_q + src * 32 + 16 * half);
+    for (int i = 0; i < S::kUnits; ++i) {
+      // (16-row tiles have fewer units than threads: the extra threads
+      // repeat the last unit, branch-free)
+      const int u = min(t + 256 * i, S::kUnitCount - 1);
+      const int sub = u % S::kRowUnits, row = u / S::kRowUnits % BM, pl = u / S::kRowUnits / BM;
+      src[i] = ((uint32_t)pl * M + min(m0 + row, M - 1)) * (16 * S::kRowUnits) + 16 * sub;
+      dst[i] = pl * S::kPlaneStride + sub * S::kUnitStride + row * 16;
+    }
+    const int ts = t % (S::SG * BM);  // threads past SG * BM repeat another's scale
+    msrc = ((uint32_t)(ts / BM) * M + min(m0 + ts % BM, M - 1)) * sizeof(ActMeta);
+    mdst = S::kActBytes + ts * 4;
   }
-  const int ts = t % (4 * BM);  // threads past 4 BM repeat another's scale
-  const int j = ts / BM, row = ts % BM;
-  r.sc = p.act_meta[(size_t)(4 * kq + j) * M + min(m0 + row, M - 1)].scale;
-  return r;
-}
-
-template <int D, int BM>
-__device__ __forceinline__ void act_store(unsigned char *buf, const ActRegs<D, BM> &r) {
-  const int t = threadIdx.x;
+  // the stage that starts at group g
+  __device__ __forceinline__ ActRegs load(const GemvArgs &p, int g) const {
+    ActRegs r;
+    const char *q = (const char *)p.act_q + (size_t)g * p.M * plane_group_bytes(D);
+    const char *mp = (const char *)(p.act_meta + (size_t)g * p.M);
 #pragma unroll
-  for (int i = 0; i < ActStage<D, BM>::kUnits; ++i)
-    ((uint4 *)buf)[min(t + 256 * i, ActStage<D, BM>::kUnitCount - 1)] = r.at(i);
-  // (duplicates store the same value to the same slot: no branch)
-  ((float *)(buf + ActStage<D, BM>::kActBytes))[t % (4 * BM)] = r.sc;
+    for (int i = 0; i < S::kUnits; ++i) r.at(i) = *(const uint4 *)(q + src[i]);
+    r.sc = *(const float *)(mp + msrc);
+    return r;
+  }
+  __device__ __forceinline__ void store(unsigned char *buf, ActRegs &r) const {
+#pragma unroll
+    for (int i = 0; i < S::kUnits; ++i) *(uint4 *)(buf + dst[i]) = r.at(i);
+    *(float *)(buf + mdst) = r.sc;
+  }
+};
+
+// A value the compiler may not see through: keeps a converted fp16 scale in
+// its own f32 register instead of folded into v_fma_mix_f32, which issues at
+// half the rate of v_fma_f32 (4.7 against 2.8 cycles).
+static __device__ __forceinline__ float opaque(float v) {
+  asm("" : "+v"(v));
+  return v;
 }
 
-// kRB: 16-row weight blocks per wave (1, 2 or 4; the workgroup covers 4 kRB);
-// BM: activation rows per workgroup (16, 32 or 64). The K quads are split over
+// A lane offset the compiler may not widen outside the loop: loads then take a
+// scalar base and this one register (a 64-bit address pair per load otherwise).
+static __device__ __forceinline__ uint32_t here(uint32_t v) {
+  asm("" : "+v"(v));
+  return v;
+}
+
+// kRB: 16-row weight blocks per wave (1 or 2; the workgroup covers 4 kRB);
+// BM: activation rows per workgroup (16 or 32). The K quads are split over
 // blockIdx.y (ks_count splits); with part set each split writes its partial
 // sums to part [ks_count][M][N] (no epilogue; a finishing kernel runs it),
 // unless fold: then the splits of a tile meet at p.splitk_counters and the
 // last to arrive runs the epilogue (the SwiGLU plane emission included).
+// Lane (c, n) of a 16 x 16 output tile (row block i, row tile mt) holds rows
+// 16 mt + 4 c + r of column n.
 template <int D, int kRB, int BM>
-__global__ __launch_bounds__(256, kRB == 4 ? 2 : kRB == 2 ? 4 : 5) void gemm_kernel(GemvArgs p, int m_tiles,
-                                                                     int ks_count, float *part,
-                                                                     int fold) {
+__global__ __launch_bounds__(256, kRB == 2 ? 4 : 5) void gemm_kernel(
+    GemvArgs p, int m_tiles, int ks_count, float *part, int fold) {
   using S = ActStage<D, BM>;
   constexpr int MT = BM / 16;         // 16-row activation tiles per wave
   constexpr int kNBW = kWaves * kRB;  // weight row blocks per workgroup
-  __shared__ __align__(16) unsigned char lds[2 * S::kBufBytes];
+  constexpr int NO = 32 * kRB;        // SwiGLU outputs per workgroup and row
+  constexpr int kStageBytes = BM * NO * 4, kParkBytes = MT * 4 * 256 * 4;
+  constexpr int kLds = 2 * S::kBufBytes > kStageBytes ? 2 * S::kBufBytes : kStageBytes;
+  __shared__ __align__(16) unsigned char lds[kLds > kParkBytes ? kLds : kParkBytes];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // uniform
   const int n_local = lane & 15, c = lane >> 4;
@@ -144,6 +174,10 @@ __global__ __launch_bounds__(256, kRB == 4 ? 2 : kRB == 2 ? 4 : 5) void gemm_ker
   // this split's quads kq0 .. kq0 + nq - 1
   const int kq0 = (int)(((long)blockIdx.y * KQ) / ks_count);
   const int nq = (int)(((long)(blockIdx.y + 1) * KQ) / ks_count) - kq0;
+  const auto row_of = [&](int mt, int r) {
+    return m0 + 16 * mt + 4 * c + r;
+  };
+  const auto block_of = [&](int i) { return nb0 + i; };
 
   // weight slots of this wave's row blocks: one per-lane base pointer plus
   // uniform tile offsets (row blocks past NB are clamped into range, compute
@@ -164,18 +198,20 @@ __global__ __launch_bounds__(256, kRB == 4 ? 2 : kRB == 2 ? 4 : 5) void gemm_ker
       sb[u][rb] = spp[toff[rb] + (size_t)q * 64];
     }
   }
-  act_store<D, BM>(lds, act_load<D, BM>(p, kq0, m0));
+  const ActMap<D, BM> map(p.M, m0);
+  {
+    ActRegs r = map.load(p, 4 * kq0);
+    map.store(lds, r);
+  }
   __syncthreads();
 
   float acc[kRB][MT][4];
 #pragma unroll
-  for (int rb = 0; rb < kRB; ++rb)
+  for (int i = 0; i < kRB; ++i)
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) acc[rb][mt][r] = 0.0f;
-  const v4i magic = {kMagic, kMagic, kMagic, kMagic};
-  const v4i zero = {0, 0, 0, 0};
+      for (int r = 0; r < 4; ++r) acc[i][mt][r] = 0.0f;
 
   for (int q0 = 0; q0 < nq; q0 += kU) {
 #pragma unroll
@@ -198,67 +234,78 @@ __global__ __launch_bounds__(256, kRB == 4 ? 2 : kRB == 2 ? 4 : 5) void gemm_ker
         wb[u][rb] = load_stream(cp + toff[rb] + (size_t)qn * 64);
         sb[u][rb] = spp[toff[rb] + (size_t)qn * 64];
       }
-      // the next quad's activations, in flight while this one computes
-      // (the last quad stages a copy of itself into the idle buffer)
-      const ActRegs<D, BM> nxt = act_load<D, BM>(p, kq0 + min(q + 1, nq - 1), m0);
-
-      // q0 is even, so this quad's buffer is u: constant LDS offsets
-      const unsigned char *buf = lds + u * S::kBufBytes;
-      uint4 wt[kRB];
-      float ws[kRB][4];  // [row block][group]: scale of this lane's column
+      // MFMA operand words of the quad's groups and the scales of this
+      // lane's columns
+      uint32_t wt[kRB][4];
+      float ws[kRB][4];
 #pragma unroll
-      for (int rb = 0; rb < kRB; ++rb) wt[rb] = quad_transpose(wc[rb]);
-#pragma unroll
-      for (int h = 0; h < (kRB + 1) / 2; ++h) {
+      for (int rb = 0; rb < kRB; ++rb) {
+        const uint4 t4 = quad_transpose(wc[rb]);
+        wt[rb][0] = t4.x;
+        wt[rb][1] = t4.y;
+        wt[rb][2] = t4.z;
+        wt[rb][3] = t4.w;
+      }
+      {
         // two row blocks' u16 scales per register, all four groups' rows
         uint32_t g4[4];
-        const uint32_t hi = 2 * h + 1 < kRB ? sc[min(2 * h + 1, kRB - 1)] << 16 : 0u;
-        column_gather((sc[2 * h] & 0xFFFFu) | hi, g4);
+        column_gather((sc[0] & 0xFFFFu) | (kRB > 1 ? sc[kRB - 1] << 16 : 0u), g4);
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-          ws[2 * h][j] = h2f(g4[j] & 0xFFFFu);
-          if (2 * h + 1 < kRB) ws[min(2 * h + 1, kRB - 1)][j] = h2f(g4[j] >> 16);
+          ws[0][j] = opaque(h2f(g4[j] & 0xFFFFu));
+          if (kRB > 1) ws[kRB - 1][j] = opaque(h2f(g4[j] >> 16));
         }
       }
+      // this quad's buffer (q0 is even, so u: constant LDS offsets) and, into
+      // the other one, the next quad's activations, loaded while this one
+      // computes (the last quad stages a copy of itself)
+      ActRegs nxt = map.load(p, 4 * (kq0 + min(q + 1, nq - 1)));
+      const unsigned char *buf = lds + u * S::kBufBytes;
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
+        const unsigned char *gb = buf + j * S::kPlanes * S::kPlaneStride;
+        const unsigned char *sb4 = buf + S::kActBytes + j * BM * 4;
         long bw[kRB];
+        v8h bh[kRB];
 #pragma unroll
-        for (int rb = 0; rb < kRB; ++rb) {
-          const uint32_t w = j == 0 ? wt[rb].x : j == 1 ? wt[rb].y : j == 2 ? wt[rb].z : wt[rb].w;
-          bw[rb] = signed_codes(w);
+        for (int i = 0; i < kRB; ++i) {
+          if constexpr (D == kPlanesQ8) bw[i] = signed_codes(wt[i][j]);
+          else bh[i] = half_codes(wt[i][j]);
         }
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
-          long av[D];
-#pragma unroll
-          for (int d = 0; d < D; ++d)
-            av[d] = *(const long *)(buf + (((j * D + d) * BM + mt * 16 + n_local) * 32 + 8 * c));
-          const float4 as4 = *(const float4 *)(buf + S::kActBytes + (j * BM + mt * 16 + 4 * c) * 4);
+          const float4 as4 = *(const float4 *)(sb4 + (16 * mt + 4 * c) * 4);
           const float as[4] = {as4.x, as4.y, as4.z, as4.w};
+          if constexpr (D == kPlanesQ8) {
+            const long av = *(const long *)(gb + (c >> 1) * S::kUnitStride +
+                                            (16 * mt + n_local) * 16 + 8 * (c & 1));
+            const v4i magic = {kMagic, kMagic, kMagic, kMagic};
 #pragma unroll
-          for (int rb = 0; rb < kRB; ++rb) {
-            if constexpr (D == 1) {
-              const v4i dd = __builtin_amdgcn_mfma_i32_16x16x32_i8(av[0], bw[rb], magic, 0, 0, 0);
-              const float wcorr = -kMagicF * ws[rb][j];
-#pragma unroll
-              for (int r = 0; r < 4; ++r) {
-                const float t = fmaf(__int_as_float(dd[r]), ws[rb][j], wcorr);
-                acc[rb][mt][r] = fmaf(t, as[r], acc[rb][mt][r]);
-              }
-            } else {
-              v4i dd[D];
-#pragma unroll
-              for (int d = 0; d < D; ++d)
-                dd[d] = __builtin_amdgcn_mfma_i32_16x16x32_i8(av[d], bw[rb], zero, 0, 0, 0);
+            for (int i = 0; i < kRB; ++i) {
+              const v4i dd = __builtin_amdgcn_mfma_i32_16x16x32_i8(av, bw[i], magic, 0, 0, 0);
+              const float wcorr = -kMagicF * ws[i][j];
 #pragma unroll
               for (int r = 0; r < 4; ++r) {
-                int T = dd[0][r];
-#pragma unroll
-                for (int d = 1; d < D; ++d) T = (T << 7) + dd[d][r];
-                acc[rb][mt][r] = fmaf((float)T * ws[rb][j], as[r], acc[rb][mt][r]);
+                const float t = fmaf(__int_as_float(dd[r]), ws[i][j], wcorr);
+                acc[i][mt][r] = fmaf(t, as[r], acc[i][mt][r]);
               }
             }
+          } else {
+            const unsigned char *ab = gb + c * S::kUnitStride + (16 * mt + n_local) * 16;
+            const v8h ahi = *(const v8h *)ab, alo = *(const v8h *)(ab + S::kPlaneStride);
+            v4f dd[kRB];
+#pragma unroll
+            for (int i = 0; i < kRB; ++i)
+              dd[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ahi, bh[i], v4f{0.f, 0.f, 0.f, 0.f}, 0,
+                                                             0, 0);
+#pragma unroll
+            for (int i = 0; i < kRB; ++i)
+              dd[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(alo, bh[i], dd[i], 0, 0, 0);
+#pragma unroll
+            for (int i = 0; i < kRB; ++i)
+#pragma unroll
+              for (int r = 0; r < 4; ++r)
+                acc[i][mt][r] = fmaf(dd[i][r] * ws[i][j], as[r], acc[i][mt][r]);
           }
           // one activation tile's MFMAs at a time: their results are
           // consumed before the next tile's are issued (register budget)
@@ -267,17 +314,13 @@ __global__ __launch_bounds__(256, kRB == 4 ? 2 : kRB == 2 ? 4 : 5) void gemm_ker
       }
       // publish the next quad's activations (the other buffer was last read
       // before the previous barrier)
-      act_store<D, BM>(lds + (u ^ 1) * S::kBufBytes, nxt);
+      map.store(lds + (u ^ 1) * S::kBufBytes, nxt);
       __syncthreads();
     }
   }
 
-  // Lane (c, n) holds rows m0 + 16 mt + 4c + r of column 16 nb + n.
-  // (the fold's publication is compiled into tiles of up to 32 rows only: in
-  // the 64-row prompt-chunk tiles its registers would spill the whole
-  // kernel; those fold only without a K split, where the sums are complete)
   if (fold) {
-    if (BM <= 32 && ks_count > 1) {
+    if (ks_count > 1) {
       // Publish this split's partial sums; the tile's last split to arrive
       // adds every split's in split order (the finishing kernel's order, so
       // the sums are the same) and runs the epilogue. The publication is the
@@ -288,14 +331,14 @@ __global__ __launch_bounds__(256, kRB == 4 ? 2 : kRB == 2 ? 4 : 5) void gemm_ker
       const size_t MN = (size_t)p.M * p.N;
       float *dst = part + (size_t)blockIdx.y * MN;
 #pragma unroll
-      for (int rb = 0; rb < kRB; ++rb)
+      for (int i = 0; i < kRB; ++i)
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
-            const int m = m0 + 16 * mt + 4 * c + r, nb = nb0 + rb;
+            const int m = row_of(mt, r), nb = block_of(i);
             if (m < p.M && nb < NB)
-              __hip_atomic_store(dst + (size_t)m * p.N + nb * 16 + n_local, acc[rb][mt][r],
+              __hip_atomic_store(dst + (size_t)m * p.N + nb * 16 + n_local, acc[i][mt][r],
                                  __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
           }
       __builtin_amdgcn_s_waitcnt(0);
@@ -311,7 +354,7 @@ __global__ __launch_bounds__(256, kRB == 4 ? 2 : kRB == 2 ? 4 : 5) void gemm_ker
       // one (row block, row tile) at a time: its up to kFoldSplits splits'
       // loads issued together, then added in split order
 #pragma unroll
-      for (int rb = 0; rb < kRB; ++rb)
+      for (int i = 0; i < kRB; ++i)
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
           float v[kFoldSplits][4];
@@ -319,7 +362,7 @@ __global__ __launch_bounds__(256, kRB == 4 ? 2 : kRB == 2 ? 4 : 5) void gemm_ker
           for (int sp = 0; sp < kFoldSplits; ++sp)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-              const int m = m0 + 16 * mt + 4 * c + r, nb = nb0 + rb;
+              const int m = row_of(mt, r), nb = block_of(i);
               const size_t idx = m < p.M && nb < NB ? (size_t)m * p.N + nb * 16 + n_local : 0;
               v[sp][r] = sp < ks_count ? __hip_atomic_load(part + sp * MN + idx, __ATOMIC_RELAXED,
                                                            __HIP_MEMORY_SCOPE_AGENT)
@@ -331,63 +374,57 @@ __global__ __launch_bounds__(256, kRB == 4 ? 2 : kRB == 2 ? 4 : 5) void gemm_ker
 #pragma unroll
             for (int sp = 1; sp < kFoldSplits; ++sp)
               if (sp < ks_count) tot += v[sp][r];
-            acc[rb][mt][r] = tot;
+            acc[i][mt][r] = tot;
           }
         }
       if (threadIdx.x == 0)
         __hip_atomic_store(p.splitk_counters + blockIdx.x, 0u, __ATOMIC_RELAXED,
                            __HIP_MEMORY_SCOPE_AGENT);
     }
-    if constexpr (BM * 32 * kRB * 4 <= 2 * S::kBufBytes) {
-      if (p.epi == EPI_SWIGLU && p.out_q) {
-        // The SwiGLU plane emission of splitk_swiglu_emit_kernel for this
-        // tile: its 4 kRB row blocks hold 32 kRB SwiGLU outputs (kRB whole
-        // quantisation groups) of each activation row; silu(g) * u into LDS
-        // [BM][32 kRB], then a half-wave quantises each (row, group).
-        constexpr int NO = 32 * kRB;
-        float *stage = (float *)lds;
-        __syncthreads();  // the staging buffers were last read before the loop's end
+    if (p.epi == EPI_SWIGLU && p.out_q) {
+      // The SwiGLU plane emission of splitk_swiglu_emit_kernel for this
+      // tile: its 4 kRB row blocks hold 32 kRB SwiGLU outputs (kRB whole
+      // quantisation groups) of each activation row; silu(g) * u into LDS
+      // [BM][32 kRB], then a half-wave quantises each (row, group).
+      float *stage = (float *)lds;
+      __syncthreads();  // the staging buffers were last read before the loop's end
 #pragma unroll
-        for (int rb = 0; rb < kRB; ++rb)
+      for (int i = 0; i < kRB; ++i)
 #pragma unroll
-          for (int mt = 0; mt < MT; ++mt)
+        for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-              const float tot = acc[rb][mt][r];
-              const float partner = row_xor8(tot);
-              if (n_local < 8)
-                stage[(16 * mt + 4 * c + r) * NO + (wave * kRB + rb) * 8 + n_local] =
-                    silu_mul(tot, partner);
-            }
-        __syncthreads();
-        const int No = p.N >> 1;
-        const int half = threadIdx.x >> 5, hl = threadIdx.x & 31;
-        for (int it = half; it < BM * kRB; it += 8) {
-          const int row = it / kRB, gl = it % kRB, m = m0 + row;
-          const int o = (n_tile * kNBW) * 8 + gl * 32 + hl;  // SwiGLU output index
-          if (m >= p.M || o >= No) continue;  // whole half-waves: No is a multiple of 32
-          const float v = stage[row * NO + gl * 32 + hl];
-          if (p.y) p.y[(size_t)m * No + o] = v;
-          if (p.out_D == 1)
-            quantize_group<1>(v, hl, o >> 5, m, p.M, p.out_q, p.out_meta);
-          else
-            quantize_group<3>(v, hl, o >> 5, m, p.M, p.out_q, p.out_meta);
-        }
-        return;
+          for (int r = 0; r < 4; ++r) {
+            const float tot = acc[i][mt][r];
+            const float partner = row_xor8(tot);
+            if (n_local < 8)
+              stage[(row_of(mt, r) - m0) * NO + (block_of(i) - n_tile * kNBW) * 8 + n_local] =
+                  silu_mul(tot, partner);
+          }
+      __syncthreads();
+      const int No = p.N >> 1;
+      const int half = threadIdx.x >> 5, hl = threadIdx.x & 31;
+      for (int it = half; it < BM * kRB; it += 8) {
+        const int row = it / kRB, gl = it % kRB, m = m0 + row;
+        const int o = (n_tile * kNBW) * 8 + gl * 32 + hl;  // SwiGLU output index
+        if (m >= p.M || o >= No) continue;  // whole half-waves: No is a multiple of 32
+        const float v = stage[row * NO + gl * 32 + hl];
+        if (p.y) p.y[(size_t)m * No + o] = v;
+        quantize_group_d(p.out_D, v, hl, o >> 5, m, p.M, p.out_q, p.out_meta);
       }
+      return;
     }
   } else if (part) {
     // split K (or a finishing pass that emits planes): this split's partial
     // sums, part[split][m][n]
     float *dst = part + (size_t)blockIdx.y * p.M * p.N;
 #pragma unroll
-    for (int rb = 0; rb < kRB; ++rb)
+    for (int i = 0; i < kRB; ++i)
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const int m = m0 + 16 * mt + 4 * c + r, nb = nb0 + rb;
-          if (m < p.M && nb < NB) dst[(size_t)m * p.N + nb * 16 + n_local] = acc[rb][mt][r];
+          const int m = row_of(mt, r), nb = block_of(i);
+          if (m < p.M && nb < NB) dst[(size_t)m * p.N + nb * 16 + n_local] = acc[i][mt][r];
         }
     return;
   }
@@ -396,21 +433,413 @@ __global__ __launch_bounds__(256, kRB == 4 ? 2 : kRB == 2 ? 4 : 5) void gemm_ker
   // column (the staging buffers are free after the last barrier): unrolled
   // over the large inlined epilogue it would index the accumulators
   // dynamically and push them to scratch.
-  static_assert(MT * 4 * 256 * 4 <= 2 * S::kBufBytes, "parking area");
   const bool paired = p.epi == EPI_SWIGLU || p.epi == EPI_QKV;
   float *park = (float *)lds + threadIdx.x;
 #pragma unroll
-  for (int rb = 0; rb < kRB; ++rb) {
+  for (int i = 0; i < kRB; ++i) {
+    const int nb = block_of(i);
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) park[(mt * 4 + r) * 256] = acc[rb][mt][r];
-    const int nb = nb0 + rb;
+      for (int r = 0; r < 4; ++r) park[(mt * 4 + r) * 256] = acc[i][mt][r];
 #pragma unroll 1
-    for (int i = 0; i < MT * 4; ++i) {
-      const float tot = park[i * 256];
+    for (int k = 0; k < MT * 4; ++k) {
+      const float tot = park[k * 256];
       const float partner = paired ? row_xor8(tot) : 0.0f;
-      const int m = m0 + 16 * (i >> 2) + 4 * c + (i & 3);
+      const int m = row_of(k >> 2, k & 3);
+      if (m < p.M && nb < NB)
+        store_output(p, p.epi, nb, n_local, m, tot, partner, epi_load(p, p.epi, nb, n_local, m));
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Prompt chunks (more than 32 rows): BM x 128 output tiles by 8 waves, both
+// operands in LDS.
+//
+// Bound: vector issue. Per output and group two f32 operations (scale by ws,
+// then by as into the running sum) against one MFMA worth 1/128 of its time;
+// MFMAs and vector work add up on this chip (a 32x32x32 i8 MFMA alone 35
+// cycles, 32 fmas alone 86, together 106), f32 operations issue at 2.4-2.9
+// cycles when at least two waves of a SIMD are ready and all operands are
+// plain vector registers (v_fma_mix_f32, conversions and scalar operands
+// 4.4-4.9), a single wave at 5-8. Hence:
+//   * the workgroup unpacks each quad's codes once (one 32-code slot, or one
+//     word, per thread) into LDS operands every wave reads, so unpacking
+//     costs 1/BM of an output instead of 1/(rows of a wave);
+//   * at most 128 registers: four waves a SIMD, two workgroups a CU;
+//   * Q8 on 32 x 32 x 32 MFMAs (half the time of 16 x 16 ones, whose K of 32
+//     leaves half the multipliers idle), split-16 on 16 x 16 x 32;
+//   * results are scaled by ws in one run and added in another (a dependent
+//     instruction right behind costs the double rate).
+// Stage: Q8 a quad, split-16 a group, double buffered, one barrier a stage.
+// ---------------------------------------------------------------------------
+constexpr int kTileThreads = 512;
+constexpr int kTileN = 128;  // columns: 8 row blocks
+
+template <int D, int BM>
+struct TileStage {
+  static constexpr bool Q8 = D == kPlanesQ8;
+  static constexpr int SG = Q8 ? 4 : 1;                   // groups per stage
+  static constexpr int kRowUnits = Q8 ? 2 : 4;            // 16-byte units per plane row
+  static constexpr int kPlanes = Q8 ? 1 : 2;              // planes per group
+  static constexpr int kPad = Q8 ? 64 : 32;               // staging writes of 8 lanes: distinct banks
+  static constexpr int kBufs = Q8 ? 2 : 3;
+  static constexpr int kAUnit = BM * 16 + kPad, kAPlane = kRowUnits * kAUnit;
+  static constexpr int kBUnit = kTileN * 16 + kPad, kBPlane = kRowUnits * kBUnit;
+  static constexpr int kB = SG * kPlanes * kAPlane;       // weight operands
+  static constexpr int kAs = kB + SG * kBPlane;           // activation scales [SG][BM]
+  static constexpr int kWs = kAs + SG * BM * 4;           // weight scales [SG][128]
+  static constexpr int kBufBytes = kWs + SG * kTileN * 4;
+  static constexpr int kUnits = SG * kPlanes * BM * kRowUnits / kTileThreads;  // per thread
+  static constexpr int kScales = SG * BM;                 // threads past it repeat others'
+};
+
+template <int D, int BM>
+__global__ __launch_bounds__(kTileThreads, 4) void gemm_tile_kernel(GemvArgs p, int m_tiles,
+                                                                    int n_tiles, int ks_count,
+                                                                    float *part, int fold) {
+  using S = TileStage<D, BM>;
+  constexpr bool Q8 = D == kPlanesQ8;
+  constexpr int WM = BM / 32, WN = 8 / WM;      // waves in M (32 rows each) and N
+  constexpr int NC = kTileN / WN;               // columns per wave
+  constexpr int TS = Q8 ? 32 : 16;              // output tile size
+  constexpr int NI = NC / TS, MT = 32 / TS, NR = TS * TS / 64;
+  constexpr int kStageBytes = BM * (kTileN / 2) * 4, kParkBytes = 16 * kTileThreads * 4;
+  constexpr int kLds0 = S::kBufs * S::kBufBytes > kStageBytes ? S::kBufs * S::kBufBytes : kStageBytes;
+  __shared__ __align__(16) unsigned char lds[kLds0 > kParkBytes ? kLds0 : kParkBytes];
+  const int t = threadIdx.x, lane = t & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int n_local = lane & 15, c = lane >> 4;
+  const int wm = wave % WM, wn = wave / WM;
+  const int KQ = p.K >> 7, NB = p.N >> 4;
+  // Block order: XCD x (block b runs on XCD b % 8) takes a contiguous run of
+  // logical blocks, row tiles fastest in bands of kBand, so the workgroups that
+  // run together on an XCD (about 64) read each operand's bytes about equally
+  // often past its L2 (a Q8 row is 1.125 bytes a column, a split-16 one 4.25,
+  // a weight 0.56).
+  const int nblk = gridDim.x, b = blockIdx.x;
+  const int xcd = b & 7;
+  const int logical = xcd * (nblk >> 3) + min(xcd, nblk & 7) + (b >> 3);
+  constexpr int kBand = Q8 ? 8 : 4;
+  const int band = logical / (kBand * n_tiles), in_band = logical - band * kBand * n_tiles;
+  const int band_rows = min(kBand, m_tiles - kBand * band);
+  const int n_tile = in_band / band_rows, m_tile = kBand * band + in_band % band_rows;
+  const int m0 = m_tile * BM, nb_wg = n_tile * 8;
+  const int kq0 = (int)(((long)blockIdx.y * KQ) / ks_count);
+  const int nq = (int)(((long)(blockIdx.y + 1) * KQ) / ks_count) - kq0;
+  const auto row_of = [&](int mt, int r) {
+    return m0 + 32 * wm + (Q8 ? 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3) : 16 * mt + 4 * c + r);
+  };
+  const auto block_of = [&](int i) {
+    return nb_wg + wn * (NC / 16) + (Q8 ? 2 * i + (c & 1) : i);
+  };
+
+  // staging: this thread's activation units (unit i lies kPlaneStep planes
+  // after unit 0, or at the same place of a taller tile's next rows) and scale
+  constexpr int kSpan = kTileThreads / S::kRowUnits;  // rows a pass covers
+  static_assert(kSpan % BM == 0, "whole planes per pass");
+  constexpr int kPlaneStep = kSpan / BM;
+  const int sub = t % S::kRowUnits, arow = t / S::kRowUnits % BM, apl = t / S::kRowUnits / BM;
+  const uint32_t asrc =
+      ((uint32_t)apl * p.M + min(m0 + arow, p.M - 1)) * (16 * S::kRowUnits) + 16 * sub;
+  const uint32_t adst = apl * S::kAPlane + sub * S::kAUnit + arow * 16;
+  const uint32_t astep = (uint32_t)kPlaneStep * p.M * (16 * S::kRowUnits);  // uniform
+  const int ts = t % S::kScales;
+  const uint32_t ssrc = ((uint32_t)(ts / BM) * p.M + min(m0 + ts % BM, p.M - 1)) * sizeof(ActMeta);
+  // ... and weight slot: wave w stages row block nb_wg + w (clamped into
+  // range: computed on a copy, never stored). Q8: lane 16 j + n unpacks
+  // group j of row n; split-16: lane 16 w + n word w of row n, for each group
+  // of the quad in turn.
+  const size_t tile0 = ((size_t)min(nb_wg + wave, NB - 1) * KQ + kq0) * 64;
+  const char *wbase = (const char *)(p.codes + tile0);
+  const char *sbase = (const char *)((const uint16_t *)p.scales + tile0);
+  const uint32_t woff = Q8 ? lane * 16 : n_local * 16 + c * 4, scoff = 2 * (Q8 ? lane : n_local);
+  // (named native vectors: HIP's uint4 class or an array of them was kept in
+  // scratch memory, whose stores waited for the loads)
+  static_assert(S::kUnits <= 2, "two units per thread");
+  v4u a0, a1, b0, b1;  // two stages' units
+  float asc, bsc;
+  v4u wreg;                 // Q8: this thread's slot
+  uint32_t aw, bw, aws, bws;  // split-16: a stage's code word; either: weight scale
+  const auto load_acts = [&](v4u &v0, v4u &v1, float &sc, int g) {
+    const char *q = (const char *)p.act_q + (size_t)g * p.M * plane_group_bytes(D);
+    const uint32_t ao = here(asrc);
+    v0 = *(const v4u *)(q + ao);
+    if constexpr (S::kUnits > 1) v1 = *(const v4u *)(q + astep + ao);
+    sc = *(const float *)((const char *)(p.act_meta + (size_t)g * p.M) + here(ssrc));
+  };
+  const auto load_slot = [&](int q) {
+    wreg = *(const v4u *)(wbase + (size_t)q * 1024 + here(woff));
+    aws = *(const uint16_t *)(sbase + (size_t)q * 128 + here(scoff));
+  };
+  const auto load_word = [&](uint32_t &w, uint32_t &sc, int g) {
+    w = *(const uint32_t *)(wbase + (size_t)g * 256 + here(woff));
+    sc = *(const uint16_t *)(sbase + (size_t)g * 32 + here(scoff));
+  };
+  const auto store_stage = [&](unsigned char *buf, v4u v0, v4u v1, float as, v4u w, uint32_t word,
+                               uint32_t sc) {
+    *(v4u *)(buf + adst) = v0;
+    if constexpr (S::kUnits > 1) *(v4u *)(buf + kPlaneStep * S::kAPlane + adst) = v1;
+    *(float *)(buf + S::kAs + ts * 4) = as;
+    const int col = 16 * wave + n_local;
+    if constexpr (Q8) {
+      const v2l lo = {signed_codes(w.x), signed_codes(w.y)};
+      const v2l hi = {signed_codes(w.z), signed_codes(w.w)};
+      unsigned char *d = buf + S::kB + c * S::kBPlane + col * 16;
+      *(v2l *)d = lo;
+      *(v2l *)(d + S::kBUnit) = hi;
+      *(float *)(buf + S::kWs + (c * kTileN + col) * 4) = h2f(sc);
+    } else {
+      *(v8h *)(buf + S::kB + c * S::kBUnit + col * 16) = half_codes(word);
+      *(float *)(buf + S::kWs + col * 4) = h2f(sc);
+    }
+  };
+
+  float acc[NI][MT][NR];
+#pragma unroll
+  for (int i = 0; i < NI; ++i)
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+      for (int r = 0; r < NR; ++r) acc[i][mt][r] = 0.0f;
+
+  // Q8: one group into the running sums. Its operands (av, bv, ws) were read
+  // by the group before it; the next group's (of `nbuf`, if any) are requested
+  // when this group's last MFMA has been issued, two runs of f32 work before
+  // they are needed.
+  const int h32 = lane >> 5, l32 = lane & 31;
+  v4i av, bv[NI];
+  float wsv[NI];
+  const auto operand_b = [&](const unsigned char *buf, int gl, int i) {
+    bv[i] = *(const v4i *)(buf + S::kB + gl * S::kBPlane + h32 * S::kBUnit +
+                           (wn * NC + 32 * i + l32) * 16);
+    wsv[i] = *(const float *)(buf + S::kWs + (gl * kTileN + wn * NC + 32 * i + l32) * 4);
+  };
+  const auto operands = [&](const unsigned char *buf, int gl) {
+    av = *(const v4i *)(buf + gl * S::kAPlane + h32 * S::kAUnit + (32 * wm + l32) * 16);
+    operand_b(buf, gl, 0);
+  };
+  const auto group8 = [&](const unsigned char *buf, int gl, bool more) {
+    float4 as[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      as[k] = *(const float4 *)(buf + S::kAs + (gl * BM + 32 * wm + 8 * k + 4 * h32) * 4);
+#pragma unroll
+    for (int i = 1; i < NI; ++i) operand_b(buf, gl, i);
+    v16i magic;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) magic[r] = kMagic;
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const v16i dd = __builtin_amdgcn_mfma_i32_32x32x32_i8(av, bv[i], magic, 0, 0, 0);
+      const float ws = wsv[i], wcorr = -kMagicF * ws;
+      __builtin_amdgcn_sched_barrier(0);
+      if (i == NI - 1 && more) operands(buf, gl + 1);
+      float tt[16];
+#pragma unroll
+      for (int r = 0; r < 16; ++r) tt[r] = fmaf(__int_as_float(dd[r]), ws, wcorr);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const float a4[4] = {as[k].x, as[k].y, as[k].z, as[k].w};
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          acc[i][0][4 * k + r] = fmaf(tt[4 * k + r], a4[r], acc[i][0][4 * k + r]);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  // split-16: one staged group into the running sums. Its weight operands and
+  // its first row tile's were read by the group before it, whose last MFMAs
+  // had been issued (three buffers: the next group's is complete a barrier
+  // earlier), so LDS trips pass under the f32 runs, the staging writes and
+  // the barrier.
+  v8h hb[NI], ahi, alo;
+  const auto rows16 = [&](const unsigned char *buf, int mt) {
+    const unsigned char *ar = buf + c * S::kAUnit + (32 * wm + 16 * mt + n_local) * 16;
+    ahi = *(const v8h *)ar;
+    alo = *(const v8h *)(ar + S::kAPlane);
+  };
+  const auto operands16 = [&](const unsigned char *buf) {
+    rows16(buf, 0);
+#pragma unroll
+    for (int i = 0; i < NI; ++i)
+      hb[i] = *(const v8h *)(buf + S::kB + c * S::kBUnit + (wn * NC + 16 * i + n_local) * 16);
+  };
+  const auto group16 = [&](const unsigned char *buf, const unsigned char *next) {
+    float ws[NI];
+#pragma unroll
+    for (int i = 0; i < NI; ++i)
+      ws[i] = *(const float *)(buf + S::kWs + (wn * NC + 16 * i + n_local) * 4);
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+      const float4 as = *(const float4 *)(buf + S::kAs + (32 * wm + 16 * mt + 4 * c) * 4);
+      const float a4[4] = {as.x, as.y, as.z, as.w};
+      v4f dd[NI];
+#pragma unroll
+      for (int i = 0; i < NI; ++i)
+        dd[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(alo, hb[i], v4f{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+#pragma unroll
+      for (int i = 0; i < NI; ++i)
+        dd[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ahi, hb[i], dd[i], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      if (mt + 1 < MT) rows16(buf, mt + 1);
+      else operands16(next);
+#pragma unroll
+      for (int i = 0; i < NI; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) dd[i][r] *= ws[i];
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < NI; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[i][mt][r] = fmaf(dd[i][r], a4[r], acc[i][mt][r]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+
+  load_acts(a0, a1, asc, 4 * kq0);
+  if constexpr (Q8) {
+    load_slot(0);
+    store_stage(lds, a0, a1, asc, wreg, 0, aws);
+  } else {
+    load_word(aw, aws, 0);
+    load_acts(b0, b1, bsc, 4 * kq0 + 1);
+    load_word(bw, bws, 1);
+    store_stage(lds, a0, a1, asc, v4u{}, aw, aws);
+    store_stage(lds + S::kBufBytes, b0, b1, bsc, v4u{}, bw, bws);
+    load_acts(a0, a1, asc, 4 * kq0 + 2);
+    load_word(aw, aws, 2);
+  }
+  __syncthreads();
+  if constexpr (Q8) {
+    for (int q = 0; q < nq; ++q) {
+      // (past the end the last quad is staged again, into the idle buffer)
+      const int qn = min(q + 1, nq - 1);
+      load_acts(a0, a1, asc, 4 * (kq0 + qn));
+      load_slot(qn);
+      const unsigned char *buf = lds + (q & 1) * S::kBufBytes;
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        if (g == 0) operands(buf, 0);
+        group8(buf, g, g < 3);
+      }
+      store_stage(lds + ((q & 1) ^ 1) * S::kBufBytes, a0, a1, asc, wreg, 0, aws);
+      __syncthreads();
+    }
+  } else {
+    // a group's stage is shorter than a trip past the L2: requested three
+    // stages ahead, stored two ahead
+    int cur = 0, nxt = S::kBufBytes, far = 2 * S::kBufBytes;
+    operands16(lds);
+    const int ng = 4 * nq;
+    for (int g0 = 0; g0 < ng; g0 += 2) {
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        const int ag = min(g0 + e + 3, ng - 1);  // (past the end the last group again, never used)
+        if (e) {
+          load_acts(a0, a1, asc, 4 * kq0 + ag);
+          load_word(aw, aws, ag);
+        } else {
+          load_acts(b0, b1, bsc, 4 * kq0 + ag);
+          load_word(bw, bws, ag);
+        }
+        group16(lds + cur, lds + nxt);
+        if (e) store_stage(lds + far, b0, b1, bsc, v4u{}, bw, bws);
+        else store_stage(lds + far, a0, a1, asc, v4u{}, aw, aws);
+        const int was = cur;
+        cur = nxt;
+        nxt = far;
+        far = was;
+        __syncthreads();
+      }
+    }
+  }
+
+  if (part) {
+    // split K (or a finishing pass that emits planes): this split's partial
+    // sums, part[split][m][n]
+    float *dst = part + (size_t)blockIdx.y * p.M * p.N;
+#pragma unroll
+    for (int i = 0; i < NI; ++i)
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int r = 0; r < NR; ++r) {
+          const int m = row_of(mt, r), nb = block_of(i);
+          if (m < p.M && nb < NB) dst[(size_t)m * p.N + nb * 16 + n_local] = acc[i][mt][r];
+        }
+    return;
+  }
+  if (fold) {
+    // SwiGLU plane emission (splitk_swiglu_emit_kernel's) for this tile's
+    // 64 outputs (two quantisation groups) of each row: silu(g) * u into
+    // LDS [BM][64], then a half-wave quantises each (row, group).
+    float *stage = (float *)lds;
+#pragma unroll
+    for (int i = 0; i < NI; ++i)
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int r = 0; r < NR; ++r) {
+          const float tot = acc[i][mt][r];
+          const float partner = row_xor8(tot);
+          if (n_local < 8)
+            stage[(row_of(mt, r) - m0) * 64 + (block_of(i) - nb_wg) * 8 + n_local] =
+                silu_mul(tot, partner);
+        }
+    __syncthreads();
+    const int No = p.N >> 1, half = t >> 5, hl = t & 31;
+    for (int it = half; it < BM * 2; it += kTileThreads / 32) {
+      const int row = it >> 1, gl = it & 1, m = m0 + row;
+      const int o = nb_wg * 8 + gl * 32 + hl;  // SwiGLU output index
+      if (m >= p.M || o >= No) continue;  // whole half-waves: No is a multiple of 32
+      const float v = stage[row * 64 + gl * 32 + hl];
+      if (p.y) p.y[(size_t)m * No + o] = v;
+      quantize_group_d(p.out_D, v, hl, o >> 5, m, p.M, p.out_q, p.out_meta);
+    }
+    return;
+  }
+  if (p.epi == EPI_PLAIN) {
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const int nb = block_of(i);
+      if (nb >= NB) continue;
+      const int n = nb * 16 + n_local;
+      const float bias = p.bias ? p.bias[n] : 0.0f;
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int r = 0; r < NR; ++r) {
+          const int m = row_of(mt, r);
+          if (m < p.M) p.y[(size_t)m * p.N + n] = p.bias ? bias + acc[i][mt][r] : acc[i][mt][r];
+        }
+    }
+    return;
+  }
+  // The other epilogues run as a loop over 16 values at a time parked in this
+  // thread's own LDS column: unrolled over the large inlined epilogue they
+  // would index the accumulators dynamically and push them to scratch. The
+  // SwiGLU / RoPE partner row n ^ 8 lives in lane ^ 8.
+  const bool paired = p.epi == EPI_SWIGLU || p.epi == EPI_QKV;
+  float *park = (float *)lds + t;
+  constexpr int PT = Q8 ? 1 : 2;  // output tiles in N parked at a time
+#pragma unroll
+  for (int i0 = 0; i0 < NI; i0 += PT) {
+#pragma unroll
+    for (int i = 0; i < PT; ++i)
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int r = 0; r < NR; ++r)
+          park[((i * MT + mt) * NR + r) * kTileThreads] = acc[i0 + i][mt][r];
+#pragma unroll 1
+    for (int k = 0; k < PT * MT * NR; ++k) {
+      const float tot = park[k * kTileThreads];
+      const float partner = paired ? row_xor8(tot) : 0.0f;
+      const int nb = block_of(i0 + k / (MT * NR));
+      const int m = row_of(k / NR % MT, k % NR);
       if (m < p.M && nb < NB)
         store_output(p, p.epi, nb, n_local, m, tot, partner, epi_load(p, p.epi, nb, n_local, m));
     }
@@ -545,8 +974,7 @@ __global__ __launch_bounds__(kEmitThreads) void splitk_resid_emit_kernel(GemvArg
   }
   __syncthreads();
   const float inv = red[kEmitThreads / 64];
-  // group quantiser (int4_matmul.zig:380-398), the same arithmetic as
-  // quantize_group, over the quad's 32 values
+  // quantize_group's arithmetic over the quad's 32 values
   float v[8];
   float amax = 0.0f;
 #pragma unroll
@@ -556,45 +984,43 @@ __global__ __launch_bounds__(kEmitThreads) void splitk_resid_emit_kernel(GemvArg
   }
   amax = fmaxf(amax, quad_xor1(amax));
   amax = fmaxf(amax, quad_xor2(amax));
-  const float scale = amax / 127.0f;
-  const float inv_s = scale == 0.0f ? 0.0f : 1.0f / scale;
-  uint64_t packed[D];
+  const int g = n0 >> 5, qp = (n0 >> 3) & 3;
+  ActMeta mm;
+  if constexpr (D == kPlanesSplit16) {
+    const float inv_s = split16_scale(amax, &mm.scale);
+    v8h hi, lo;
 #pragma unroll
-  for (int d = 0; d < D; ++d) packed[d] = 0;
-  int csum = 0;
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const float yq = v[i] * inv_s;
-    float q0f = roundf(yq);
-    q0f = fminf(fmaxf(q0f, -127.0f), 127.0f);
-    int qd[3] = {(int)q0f, 0, 0};
-    if (D == 3) {
-      const float r1 = (yq - q0f) * 128.0f;
-      const float q1f = roundf(r1);
-      const float r2 = (r1 - q1f) * 128.0f;
-      qd[1] = (int)q1f;
-      qd[2] = (int)roundf(r2);
+    for (int i = 0; i < 8; ++i) {
+      const float yq = v[i] * inv_s;
+      const _Float16 hv = (_Float16)yq;
+      hi[split16_pos(i)] = hv;
+      lo[split16_pos(i)] = (_Float16)(yq - (float)hv);
     }
-    int comb = 0;
-#pragma unroll
-    for (int d = 0; d < D; ++d) {
-      packed[d] |= (uint64_t)(uint8_t)(int8_t)qd[d] << (8 * i);
-      comb = comb * 128 + qd[d];
+    mm.corr = 0;
+    if (act) {
+      v8h *q = (v8h *)p.out_q;
+      q[(((size_t)g * 2 + 0) * p.M + m) * 4 + qp] = hi;
+      q[(((size_t)g * 2 + 1) * p.M + m) * 4 + qp] = lo;
+      if (qp == 0) p.out_meta[(size_t)g * p.M + m] = mm;
     }
-    csum += comb;
-  }
-  csum += quad_xor1(csum);
-  csum += quad_xor2(csum);
-  if (act) {
-    const int g = n0 >> 5, qp = (n0 >> 3) & 3;
+  } else {
+    const float scale = amax / 127.0f;
+    const float inv_s = scale == 0.0f ? 0.0f : 1.0f / scale;
+    uint64_t packed = 0;
+    int csum = 0;
 #pragma unroll
-    for (int d = 0; d < D; ++d)
-      *(uint64_t *)(p.out_q + (((size_t)g * D + d) * p.M + m) * 32 + qp * 8) = packed[d];
-    if (qp == 0) {
-      ActMeta mm;
-      mm.scale = D == 3 ? scale * (1.0f / 16384.0f) : scale;
+    for (int i = 0; i < 8; ++i) {
+      const int q0 = (int)fminf(fmaxf(roundf(v[i] * inv_s), -127.0f), 127.0f);
+      packed |= (uint64_t)(uint8_t)(int8_t)q0 << (8 * i);
+      csum += q0;
+    }
+    csum += quad_xor1(csum);
+    csum += quad_xor2(csum);
+    if (act) {
+      *(uint64_t *)(p.out_q + ((size_t)g * p.M + m) * 32 + qp * 8) = packed;
+      mm.scale = scale;
       mm.corr = 7 * csum;
-      p.out_meta[(size_t)g * p.M + m] = mm;
+      if (qp == 0) p.out_meta[(size_t)g * p.M + m] = mm;
     }
   }
 }
@@ -603,25 +1029,29 @@ __global__ __launch_bounds__(kEmitThreads) void splitk_resid_emit_kernel(GemvArg
 
 GemmShape plan_gemm(int N, int M, int K, int D, size_t ws_floats) {
   GemmShape s;
-  const int bm = M <= 16 ? 16 : M <= 32 ? 32 : 64;
-  s.mt = bm / 16;
-  s.m_tiles = (M + bm - 1) / bm;
-  // Row blocks per wave and the workgroup target, from sweeps of the 7B
-  // shapes: 16- and 32-row tiles (decode lanes; 16 rows up to 16, so small
-  // batches do not pay for 32 rows of MFMA and scaling work) 1 row block per wave for one-digit
-  // planes, 2 for three, toward about 1024 workgroups; 64-row tiles (prompt
-  // chunks) 2 for one digit (4 workgroups per CU), 4 for three once that
-  // still fills the GPU, toward about 512.
   const int NB = N / 16, KQ = K / 128;
-  const long big = (long)s.m_tiles * ((NB + 15) / 16);
-  int target;
-  if (bm <= 32) {
-    s.nt = D == 1 ? 4 : 8;
+  int bm, target;
+  if (M <= 32) {
+    // decode lanes (16 rows up to 16, so small batches do not pay for 32 rows
+    // of MFMA and scaling work): 1 row block per wave for Q8, 2 for split-16,
+    // toward about 1024 workgroups (sweeps of the 7B shapes)
+    bm = M <= 16 ? 16 : 32;
+    s.nt = D == kPlanesQ8 ? 4 : 8;
     target = 1024;
   } else {
-    s.nt = D == 3 && big >= 384 ? 16 : 8;
-    target = 512;
+    // prompt chunks: 128-row tiles, 64-row ones where they round M up to so
+    // many fewer rows that they win (a row of theirs costs 1.2 of a 128-row
+    // tile's with Q8, 1.3 with split-16: 2048 x 18944 x 3584 454 against 390
+    // us, 1999 x 3584 x 18944 1050 against 845), toward one workgroup a CU
+    // (M = 100, 3584 x 18944: 65 us with 256, 66 with 1024; M = 200, 3584 x
+    // 3584 with 64-row tiles 25.5 against 28.4)
+    const long r64 = (M + 63) / 64 * 64, r128 = (M + 127) / 128 * 128;
+    bm = r64 * (D == kPlanesQ8 ? 12 : 13) < r128 * 10 ? 64 : 128;
+    s.nt = kTileN / 16;
+    target = 256;
   }
+  s.mt = bm / 16;
+  s.m_tiles = (M + bm - 1) / bm;
   s.n_tiles = (NB + s.nt - 1) / s.nt;
   s.grid = s.m_tiles * s.n_tiles;
   // split K over workgroups (at least 2 quads each) toward the target, as far
@@ -641,11 +1071,12 @@ size_t gemm_splitk_floats(int N, int M, int K, int D) {
 // The launch shape of these arguments (plan_gemm plus the tuning
 // overrides); false when they are invalid.
 static bool gemm_plan(const GemvArgs &a, GemmShape &s) {
-  if (a.N % 16 || a.K % 128 || a.M < 1 || !a.act_q || !a.act_meta || (a.D != 1 && a.D != 3))
+  if (a.N % 16 || a.K % 128 || a.M < 1 || !a.act_q || !a.act_meta ||
+      (a.D != kPlanesQ8 && a.D != kPlanesSplit16))
     return false;
   if (a.ss_out || a.arg_parts || a.x_in) return false;  // GEMV-only
   s = plan_gemm(a.N, a.M, a.K, a.D, a.splitk_ws ? a.splitk_ws_floats : 0);
-  if (a.rb_override == 1 || a.rb_override == 2 || a.rb_override == 4) {  // tuning
+  if (s.mt <= 2 && (a.rb_override == 1 || a.rb_override == 2)) {  // tuning
     s.nt = 4 * a.rb_override;
     s.n_tiles = (a.N / 16 + s.nt - 1) / s.nt;
     s.grid = s.m_tiles * s.n_tiles;
@@ -659,32 +1090,25 @@ static bool gemm_plan(const GemvArgs &a, GemmShape &s) {
   return true;
 }
 
-// Whether a tile of this shape stages its SwiGLU outputs for the plane
-// emission in the kernel's LDS (BM rows x 32 kRB outputs in the two
-// activation buffers).
-static bool swiglu_stage_fits(int D, const GemmShape &s) {
-  const int bm = 16 * s.mt, rb = s.nt / 4;
-  const int buf = 4 * D * bm * 32 + 4 * bm * 4;  // ActStage<D, BM>::kBufBytes
-  return bm * 32 * rb * 4 <= 2 * buf;
-}
-
 // A SwiGLU GEMM without a K split emits down's planes from its own tiles
-// (their sums are complete), with no partial sums, when the staging fits.
+// (their sums are complete), with no partial sums.
 static bool gemm_direct_emit(const GemvArgs &a, const GemmShape &s) {
-  return a.out_q && a.epi == EPI_SWIGLU && s.ks == 1 && swiglu_stage_fits(a.D, s);
+  return a.out_q && a.epi == EPI_SWIGLU && s.ks == 1;
 }
 
 // Whether the planes a launch emits overlap the planes it reads.
 static bool emit_overlaps_input(const GemvArgs &a) {
-  const size_t in_bytes = (size_t)(a.K / 32) * a.D * a.M * 32;
-  const size_t out_bytes = a.out_q ? (size_t)(a.N / 64) * a.out_D * a.M * 32 : 0;
+  const size_t in_bytes = (size_t)(a.K / 32) * plane_group_bytes(a.D) * a.M;
+  const size_t out_bytes =
+      a.out_q ? (size_t)(a.N / (a.epi == EPI_SWIGLU ? 64 : 32)) * plane_group_bytes(a.out_D) * a.M : 0;
   return a.out_q && (const int8_t *)a.out_q < a.act_q + in_bytes &&
          a.act_q < (const int8_t *)a.out_q + out_bytes;
 }
 
 bool gemm_emit_ok(const GemvArgs &a) {
   GemmShape s;
-  if (!a.out_q || !a.out_meta || (a.out_D != 1 && a.out_D != 3) || !gemm_plan(a, s)) return false;
+  if (!a.out_q || !a.out_meta || (a.out_D != kPlanesQ8 && a.out_D != kPlanesSplit16) ||
+      !gemm_plan(a, s)) return false;
   if (s.ks != 1 && s.ks != 2 && s.ks != 4 && s.ks != 8 && s.ks != 16) return false;
   if (a.epi == EPI_SWIGLU && gemm_direct_emit(a, s) && !emit_overlaps_input(a))
     return (a.N / 2) % 32 == 0;
@@ -725,14 +1149,23 @@ hipError_t launch_gemm(const GemvArgs &a, hipStream_t st) {
 #define GK_GEMM_BM(DD, RB) \
   do {                       \
     if (s.mt == 1) GK_GEMM(DD, RB, 16);                           \
-    else if (s.mt == 2) GK_GEMM(DD, RB, 32);                      \
-    else GK_GEMM(DD, RB, 64);                                     \
+    else GK_GEMM(DD, RB, 32);                                     \
   } while (0)
-  if (a.D == 1) {
-    if (s.nt == 16) GK_GEMM_BM(1, 4); else if (s.nt == 8) GK_GEMM_BM(1, 2); else GK_GEMM_BM(1, 1);
+#define GK_TILE(DD, BM)                                                                          \
+  hipLaunchKernelGGL((gemm_tile_kernel<DD, BM>), grid, dim3(kTileThreads), 0, st, a, s.m_tiles,  \
+                     s.n_tiles, s.ks, part, fold ? 1 : 0)
+  if (s.mt > 2) {
+    if (a.D == kPlanesQ8) {
+      if (s.mt == 4) GK_TILE(kPlanesQ8, 64); else GK_TILE(kPlanesQ8, 128);
+    } else {
+      if (s.mt == 4) GK_TILE(kPlanesSplit16, 64); else GK_TILE(kPlanesSplit16, 128);
+    }
+  } else if (a.D == kPlanesQ8) {
+    if (s.nt == 8) GK_GEMM_BM(kPlanesQ8, 2); else GK_GEMM_BM(kPlanesQ8, 1);
   } else {
-    if (s.nt == 16) GK_GEMM_BM(3, 4); else if (s.nt == 8) GK_GEMM_BM(3, 2); else GK_GEMM_BM(3, 1);
+    if (s.nt == 8) GK_GEMM_BM(kPlanesSplit16, 2); else GK_GEMM_BM(kPlanesSplit16, 1);
   }
+#undef GK_TILE
 #undef GK_GEMM_BM
 #undef GK_GEMM
   hipError_t e = hipGetLastError();
@@ -751,7 +1184,7 @@ hipError_t launch_gemm(const GemvArgs &a, hipStream_t st) {
   } while (0)
 #define GK_EMIT_D(KS)                                  \
   do {                                                \
-    if (a.out_D == 1) GK_EMIT(KS, 1); else GK_EMIT(KS, 3); \
+    if (a.out_D == kPlanesQ8) GK_EMIT(KS, kPlanesQ8); else GK_EMIT(KS, kPlanesSplit16); \
   } while (0)
     switch (s.ks) {
       case 1: GK_EMIT_D(1); break;

@@ -43,6 +43,30 @@ static __device__ __forceinline__ long signed_codes(uint32_t w) {
   return (long)(((uint64_t)hi << 32) | (uint64_t)lo);
 }
 
+// Eight 4-bit codes of one u32 word -> eight halves holding (u - 7) * 2^-10
+// exactly, in the order k0 k2 k4 k6 k1 k3 k5 k7 (split16_pos): a nibble at
+// bit 0 of a half is the subnormal u * 2^-24, and one packed fma scales it
+// and subtracts 7.
+typedef _Float16 v2h __attribute__((ext_vector_type(2)));
+typedef _Float16 v8h __attribute__((ext_vector_type(8)));
+static __device__ __forceinline__ v8h half_codes(uint32_t w) {
+  const v2h mul = {(_Float16)16384.0f, (_Float16)16384.0f};
+  const v2h add = {(_Float16)(-7.0f / 1024.0f), (_Float16)(-7.0f / 1024.0f)};
+  v8h r;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const v2h c = __builtin_elementwise_fma(
+        __builtin_bit_cast(v2h, (w >> (4 * i)) & 0x000F000Fu), mul, add);
+    r[2 * i] = c.x;
+    r[2 * i + 1] = c.y;
+  }
+  return r;
+}
+// Position of element k (0..31) of a group in a split-16 plane row.
+static __host__ __device__ constexpr int split16_pos(int k) {
+  return (k & ~7) | ((k & 7) >> 1) | ((k & 1) << 2);
+}
+
 // Even lanes: (own u16) | (u16 of the next lane) << 16; DPP quad_perm
 // [1, 0, 3, 2] reads the neighbour's value without a trip through LDS.
 static __device__ __forceinline__ uint32_t scale_pair(uint32_t s) {

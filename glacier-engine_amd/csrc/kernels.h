@@ -11,16 +11,25 @@
 //          Code u decodes to (u - 7) (int4_matmul.zig:22-25).
 //   scales uint16  [NB][KQ][64 lanes] = fp16 w_scale[row][g], same lane order.
 //
-// Activation digit planes (A operand of v_mfma_i32_16x16x32_i8):
-//   q      int8   [G][D][M][32]   (D = digit planes: 1 for Q8, 3 for F32)
-//   meta   {f32 scale, i32 corr} [G][M]
-//   The group dot is  (f32(T - corr) * w_scale) * scale  with
-//   T = sum_d 128^(D-1-d) * sum_k u_k * q_d[k]   (u = stored code).
+// Activation planes, one of three layouts D (G = K / 32 groups):
+//   D = 1 (Q8), 3 (f32 as three digits, for the GEMV's integer dots):
+//     q    int8   [G][D][M][32]
+//     meta {f32 scale, i32 corr} [G][M]
+//     The group dot is  (f32(T - corr) * w_scale) * scale  with
+//     T = sum_d 128^(D-1-d) * sum_k u_k * q_d[k]   (u = stored code).
+//   D = 2 (f32 as an fp16 pair, for the GEMM's fp16 MFMAs):
+//     q    fp16   [G][hi, lo][M][32], element k at split16_pos(k);
+//          hi + lo = x / 2^e to 2^-23 of x (2^e: a power of two per group)
+//     meta {f32 scale = 2^(e + 10), 0} [G][M]
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
 namespace gk {
+
+constexpr int kPlanesQ8 = 1, kPlanesSplit16 = 2, kPlanesDigits = 3;
+// Bytes of q per group and activation row.
+constexpr int plane_group_bytes(int D) { return D == kPlanesSplit16 ? 128 : 32 * D; }
 
 struct ActMeta {
   float scale;
@@ -88,7 +97,7 @@ struct GemvArgs {
   int ksplit_lds_off;       // set by launch_gemv: LDS offset of the SwiGLU plane buffer
   QkvArgs qkv;
   // EPI_SWIGLU only: also (or instead, with y == null) emit the SwiGLU output
-  // as digit planes [G][out_D][M][32] + meta [G][M] of width N/2, ready as
+  // as planes of layout out_D and width N/2, ready as
   // the next projection's input.
   int8_t *out_q;
   ActMeta *out_meta;
@@ -130,8 +139,7 @@ struct GemvArgs {
   unsigned *splitk_counters;
   int splitk_counter_count;
   // GEMM with out_q set (launch_gemm, when gemm_emit_ok): the finishing
-  // pass also writes the next projection's digit planes [G][out_D][M][32] +
-  // meta. EPI_SWIGLU: the SwiGLU outputs (width N/2); EPI_RESID: y after
+  // pass also writes the next projection's planes (layout out_D). EPI_SWIGLU: the SwiGLU outputs (width N/2); EPI_RESID: y after
   // the RMSNorm with these weights and in_eps (y itself is written too).
   const float *emit_norm_w;
 };
@@ -166,6 +174,10 @@ hipError_t launch_gemv(const GemvArgs &a, hipStream_t st);
 // (11008x4096: 12.5 us against 16.2, 18944x3584: 15.2 against 17.0;
 // 4096x4096: 8.8 against 8.2).
 constexpr int kGemvMaxRows = 2;
+// Planes layout of a projection over `rows` rows with Q8 or f32 activations.
+constexpr int planes_layout(bool q8, int rows) {
+  return q8 ? kPlanesQ8 : rows > kGemvMaxRows ? kPlanesSplit16 : kPlanesDigits;
+}
 
 // MFMA GEMM (K2) for more than kGemvMaxRows activation rows: same arguments
 // and epilogues as launch_gemv without the GEMV-only stages (partial sums of

@@ -42,8 +42,7 @@ static __device__ __forceinline__ float load_x(const void *x, int bf16, size_t i
 static __device__ __forceinline__ void emit_group(const PlanesDst &pd, float v, int hl, int g,
                                                   int m, int M) {
   if (!pd.q) return;
-  if (pd.D == 1) quantize_group<1>(v, hl, g, m, M, pd.q, pd.meta);
-  else quantize_group<3>(v, hl, g, m, M, pd.q, pd.meta);
+  quantize_group_d(pd.D, v, hl, g, m, M, pd.q, pd.meta);
 }
 
 // grid = (ceil(G / 8), M): each block converts 8 groups of one row; with a
@@ -118,6 +117,9 @@ hipError_t launch_prep_act(const void *x, int x_bf16, const float *norm_w, float
   if (D == 1)
     hipLaunchKernelGGL(prep_act_kernel<1>, grid, dim3(256), 0, st, x, x_bf16, norm_w, eps, M,
                        K, act_q, meta, normed_out);
+  else if (D == kPlanesSplit16)
+    hipLaunchKernelGGL(prep_act_kernel<kPlanesSplit16>, grid, dim3(256), 0, st, x, x_bf16, norm_w,
+                       eps, M, K, act_q, meta, normed_out);
   else
     hipLaunchKernelGGL(prep_act_kernel<3>, grid, dim3(256), 0, st, x, x_bf16, norm_w, eps, M,
                        K, act_q, meta, normed_out);
@@ -675,7 +677,7 @@ __global__ __launch_bounds__(LB) void gemv_kernel(GemvArgs a) {
 // Launch shape for these arguments; also fills the fields launch_gemv
 // derives (ksplit, LDS offsets). False when the arguments are invalid.
 static bool gemv_shape(GemvArgs &a, GemvShape &p) {
-  if (a.M < 1 || a.M > kGemvMaxRows || a.N % 16 || a.K % 128 ||
+  if (a.M < 1 || a.M > kGemvMaxRows || a.N % 16 || a.K % 128 || (a.D != 1 && a.D != 3) ||
       (!a.x_in && (!a.act_q || !a.act_meta)))
     return false;
   const bool emit_planes = a.epi == EPI_SWIGLU && a.out_q;

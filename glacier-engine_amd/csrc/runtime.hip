@@ -18,7 +18,11 @@ using gh::hip_fail;
 // GEMM's split-K partial sums. One array per GPU for the life of the
 // process; host code reaches it only through the address
 // hipGetSymbolAddress returns on that device (glacier_hip_init).
-static constexpr size_t kNoAllocPlanesBytes = 4u << 20;
+// A call's planes may take 4 MiB counted at three bytes an f32 element (the
+// GEMV's digits; 104 bytes a group with its meta); the GEMM's fp16 pairs take
+// 136, so the region holds 4 MiB * 136 / 104, rounded up.
+static constexpr size_t kNoAllocPlanesLimit = 4u << 20;
+static constexpr size_t kNoAllocPlanesBytes = 5632u << 10;
 static constexpr size_t kNoAllocSplitkBytes = 12u << 20;
 static constexpr uint32_t kNoAllocMaxRows = 64;
 static __device__ __align__(256) uint8_t scratch[kNoAllocPlanesBytes + kNoAllocSplitkBytes];
@@ -512,17 +516,19 @@ uint64_t glacier_hip_int4_weight_device_bytes(const glacier_hip_int4_weight *w) 
   return w ? w->device_bytes : 0;
 }
 
-// Activation planes: int8 [G][D][m][32] followed (256-aligned) by ActMeta [G][m].
+// Activation planes (kernels.h) followed (256-aligned) by ActMeta [G][m].
 static size_t al256(size_t b) { return (b + 255) & ~(size_t)255; }
-static size_t planes_q_bytes(uint32_t m, uint32_t in_f, int D) { return (size_t)(in_f / 32) * D * m * 32; }
+static size_t planes_q_bytes(uint32_t m, uint32_t in_f, int D) {
+  return (size_t)(in_f / 32) * gk::plane_group_bytes(D) * m;
+}
 static size_t planes_bytes(uint32_t m, uint32_t in_f, int D) {
   return al256(planes_q_bytes(m, in_f, D)) + (size_t)(in_f / 32) * m * sizeof(gk::ActMeta);
 }
 
-static int act_digits(int activation) {
-  if (activation == GLACIER_HIP_ACT_Q8) return 1;
-  if (activation == GLACIER_HIP_ACT_F32) return 3;
-  return 0;
+// Planes layout of m rows, 0 for an activation mode that has none.
+static int act_planes(int activation, uint32_t m) {
+  if (activation != GLACIER_HIP_ACT_Q8 && activation != GLACIER_HIP_ACT_F32) return 0;
+  return gk::planes_layout(activation == GLACIER_HIP_ACT_Q8, (int)std::min(m, GLACIER_HIP_MAX_ROWS));
 }
 
 // ws == null: the stream's split-K workspace, grown on demand; else the
@@ -586,7 +592,7 @@ static int gemv_common(glacier_hip_context *ctx, glacier_hip_int4_weight *w, con
   if (w->ctx != ctx) return GLACIER_HIP_INVALID_HANDLE;
   if (m == 0 || m > GLACIER_HIP_MAX_ROWS) return GLACIER_HIP_SHAPE_MISMATCH;
   if (x_dtype != GLACIER_HIP_F32 && x_dtype != GLACIER_HIP_BF16) return GLACIER_HIP_DTYPE_UNSUPPORTED;
-  const int D = act_digits(gh::resolve_activation(activation, w->out_f, w->in_f));
+  const int D = act_planes(gh::resolve_activation(activation, w->out_f, w->in_f), m);
   if (!D) return GLACIER_HIP_INVALID_ARGUMENT;
   auto &ss = ctx->per_stream[st];
   const size_t pb = planes_bytes(m, w->in_f, D);
@@ -611,6 +617,11 @@ int glacier_hip_int4_gemv(glacier_hip_context *ctx, glacier_hip_int4_weight *w, 
                      stream ? (hipStream_t)stream : ctx->stream);
 }
 
+// What a call's planes count against kNoAllocPlanesLimit.
+static size_t noalloc_planes_bytes(uint32_t m, uint32_t in_f, int D) {
+  return planes_bytes(m, in_f, D == gk::kPlanesQ8 ? D : gk::kPlanesDigits);
+}
+
 int glacier_hip_int4_gemv_noalloc(glacier_hip_context *ctx, glacier_hip_int4_weight *w,
                                   const void *x_dev, int x_dtype, uint32_t m, const float *bias_dev,
                                   float *y_dev, int activation, void *stream) {
@@ -618,10 +629,10 @@ int glacier_hip_int4_gemv_noalloc(glacier_hip_context *ctx, glacier_hip_int4_wei
   if (!w || !x_dev || !y_dev) return GLACIER_HIP_INVALID_ARGUMENT;
   if (w->ctx != ctx) return GLACIER_HIP_INVALID_HANDLE;
   if (x_dtype != GLACIER_HIP_F32 && x_dtype != GLACIER_HIP_BF16) return GLACIER_HIP_DTYPE_UNSUPPORTED;
-  const int D = act_digits(gh::resolve_activation(activation, w->out_f, w->in_f));
+  const int D = act_planes(gh::resolve_activation(activation, w->out_f, w->in_f), m);
   if (!D) return GLACIER_HIP_INVALID_ARGUMENT;
   GH_SUBMISSION(ctx);
-  if (m == 0 || m > kNoAllocMaxRows || planes_bytes(m, w->in_f, D) > kNoAllocPlanesBytes) {
+  if (m == 0 || m > kNoAllocMaxRows || noalloc_planes_bytes(m, w->in_f, D) > kNoAllocPlanesLimit) {
     ctx->last_error = "int4_gemv_noalloc: more rows than its fixed scratch holds (at most 64 "
                       "rows and 4 MiB of activation planes)";
     return GLACIER_HIP_SHAPE_MISMATCH;
@@ -639,7 +650,7 @@ int glacier_hip_int4_gemv_noalloc(glacier_hip_context *ctx, glacier_hip_int4_wei
 }
 
 uint64_t glacier_hip_activation_bytes(uint32_t m, uint32_t in_f, int activation) {
-  const int D = act_digits(activation);
+  const int D = act_planes(activation, m);
   if (!D || in_f % 128 != 0 || m == 0) return 0;
   return planes_bytes(m, in_f, D);
 }
@@ -648,7 +659,7 @@ int glacier_hip_activation_prepare(glacier_hip_context *ctx, const void *x_dev, 
                                    uint32_t m, uint32_t in_f, int activation, void *act_dev,
                                    void *stream) {
   if (!ctx || !x_dev || !act_dev) return GLACIER_HIP_INVALID_ARGUMENT;
-  const int D = act_digits(activation);
+  const int D = act_planes(activation, m);
   if (!D) return GLACIER_HIP_INVALID_ARGUMENT;
   if (m == 0 || m > GLACIER_HIP_MAX_ROWS || in_f == 0 || in_f % 128 != 0) return GLACIER_HIP_SHAPE_MISMATCH;
   if (x_dtype != GLACIER_HIP_F32 && x_dtype != GLACIER_HIP_BF16) return GLACIER_HIP_DTYPE_UNSUPPORTED;
@@ -662,7 +673,7 @@ int glacier_hip_int4_gemv_prepared(glacier_hip_context *ctx, glacier_hip_int4_we
                                    const float *bias_dev, float *y_dev, void *stream) {
   if (!ctx || !w || !act_dev || !y_dev) return GLACIER_HIP_INVALID_ARGUMENT;
   if (w->ctx != ctx) return GLACIER_HIP_INVALID_HANDLE;
-  const int D = act_digits(activation);
+  const int D = act_planes(activation, m);
   if (!D) return GLACIER_HIP_INVALID_ARGUMENT;
   if (m == 0 || m > GLACIER_HIP_MAX_ROWS) return GLACIER_HIP_SHAPE_MISMATCH;
   GH_SUBMISSION(ctx);

@@ -785,13 +785,16 @@ struct GemvPlan {
   int S;
 };
 
-int layer_D(const glacier_hip_session *s, uint32_t out_f, uint32_t in_f) {
-  return gh::resolve_activation(s->opt.layer_activation, out_f, in_f) == GLACIER_HIP_ACT_Q8 ? 1 : 3;
+// Planes layout of a layer projection / the head over `rows` rows.
+int layer_D(const glacier_hip_session *s, uint32_t out_f, uint32_t in_f, int rows) {
+  return gk::planes_layout(
+      gh::resolve_activation(s->opt.layer_activation, out_f, in_f) == GLACIER_HIP_ACT_Q8, rows);
 }
 
-int head_D(const glacier_hip_session *s) {
+int head_D(const glacier_hip_session *s, int rows) {
   const auto &c = s->model->cfg;
-  return gh::resolve_activation(s->opt.head_activation, c.vocab_size, c.dim) == GLACIER_HIP_ACT_Q8 ? 1 : 3;
+  return gk::planes_layout(
+      gh::resolve_activation(s->opt.head_activation, c.vocab_size, c.dim) == GLACIER_HIP_ACT_Q8, rows);
 }
 
 // One projection over `rows` activation rows with the given epilogue. The
@@ -998,7 +1001,7 @@ bool attn_o_usable(glacier_hip_session *s) {
                    s->step_dev->ctx_len};
   for (uint32_t l = 0; ok && l < c.num_layers; ++l) {
     const LayerDev &L = s->model->layers[l];
-    ok = layer_D(s, L.o->out_f, L.o->in_f) == 1 && L.o->out_f == c.dim &&
+    ok = layer_D(s, L.o->out_f, L.o->in_f, 1) == gk::kPlanesQ8 && L.o->out_f == c.dim &&
          gk::attn_o_ok(attn_o_args(s, rp, l, s->ss_parts)) &&
          gk::attn_o_groups((int)c.dim) <= 1024;
   }
@@ -1046,10 +1049,10 @@ hipError_t enqueue_layers(glacier_hip_session *s, int rows, const RowPtrs &rp, h
   for (uint32_t l = 0; l < c.num_layers; ++l) {
     const LayerDev &L = m->layers[l];
     q.layer = (int)l;
-    const int Dq = layer_D(s, L.qkv->out_f, L.qkv->in_f);
-    const int Do = layer_D(s, L.o->out_f, L.o->in_f);
-    const int Dg = layer_D(s, L.gu->out_f / 2, L.gu->in_f);
-    const int Dd = layer_D(s, L.down->out_f, L.down->in_f);
+    const int Dq = layer_D(s, L.qkv->out_f, L.qkv->in_f, rows);
+    const int Do = layer_D(s, L.o->out_f, L.o->in_f, rows);
+    const int Dg = layer_D(s, L.gu->out_f / 2, L.gu->in_f, rows);
+    const int Dd = layer_D(s, L.down->out_f, L.down->in_f, rows);
     // RMSNorm -> QKV (+RoPE, KV row write into the lane's page)
     ProjIn qin;
     if (x_planes) {
@@ -1195,7 +1198,7 @@ hipError_t enqueue_layers(glacier_hip_session *s, int rows, const RowPtrs &rp, h
     x_planes = false;
     if (!chain && !last) {  // GEMM: the next layer's QKV planes from down's finishing pass
       const LayerDev &N = m->layers[l + 1];
-      dout.emit = gk::PlanesDst{s->act_q, s->act_meta, layer_D(s, N.qkv->out_f, N.qkv->in_f)};
+      dout.emit = gk::PlanesDst{s->act_q, s->act_meta, layer_D(s, N.qkv->out_f, N.qkv->in_f, rows)};
       dout.emit_norm_w = N.in_norm;
       x_planes = gemm_emit_ok(s, L.down, Dd, rows, gk::EPI_RESID, din, dout);
       if (!x_planes) {
@@ -1241,12 +1244,12 @@ hipError_t enqueue_head(glacier_hip_session *s, int rows, const float *x, bool e
     out.arg_words = words;
     out.arg_word_count = W;
     out.prehead = elig && pre;
-    hipError_t e = run_proj(s, m->head, head_D(s), rows, gk::EPI_PLAIN, in, out, st);
+    hipError_t e = run_proj(s, m->head, head_D(s, rows), rows, gk::EPI_PLAIN, in, out, st);
     if (e != hipSuccess) return e;
-    const int nparts = gk::gemv_argmax_parts((int)V, (int)c.dim, rows, head_D(s));
+    const int nparts = gk::gemv_argmax_parts((int)V, (int)c.dim, rows, head_D(s, rows));
     return gk::launch_argmax_parts(out.arg_parts, nparts, V, rows, words, W, s->arg_result, st);
   }
-  hipError_t e = run_proj(s, m->head, head_D(s), rows, gk::EPI_PLAIN, in, out, st);
+  hipError_t e = run_proj(s, m->head, head_D(s, rows), rows, gk::EPI_PLAIN, in, out, st);
   if (e != hipSuccess) return e;
   return gk::launch_argmax(s->logits, V, rows, words, W, s->arg_scratch, s->arg_counters,
                            s->arg_result, st);
@@ -1857,7 +1860,7 @@ static glacier_hip_session *session_create_impl(glacier_hip_model *m,
   A((void **)&s->attn, (size_t)M * c.dim * 4);
   A((void **)&s->act, (size_t)M * c.hidden_dim * 4);
   A((void **)&s->logits, (size_t)L * c.vocab_size * 4);
-  A((void **)&s->act_q, Gmax * 3 * M * 32);
+  A((void **)&s->act_q, Gmax * M * gk::plane_group_bytes(gk::kPlanesSplit16));
   A((void **)&s->act_meta, Gmax * M * sizeof(gk::ActMeta));
   // the gate/up epilogue emits planes for every GEMV launch (up to
   // kGemvMaxRows rows) and attention the O projection's for every step of
@@ -1869,7 +1872,7 @@ static glacier_hip_session *session_create_impl(glacier_hip_model *m,
   // act_q2 also holds the O projection's planes, emitted by attention
   const size_t G2 = std::max<size_t>(c.hidden_dim, (size_t)c.num_heads * c.head_dim) / 32;
   const size_t q2_groups_rows = std::max(G2 * s->planes2_rows, (size_t)(c.dim / 32) * M);
-  A((void **)&s->act_q2, q2_groups_rows * 3 * 32);
+  A((void **)&s->act_q2, q2_groups_rows * gk::plane_group_bytes(gk::kPlanesSplit16));
   A((void **)&s->act_meta2, q2_groups_rows * sizeof(gk::ActMeta));
   A((void **)&s->att_scratch, std::max<size_t>(att, 1) * 4);
   A((void **)&s->ss_parts, (size_t)32 * 1024 * sizeof(float));
@@ -1880,7 +1883,7 @@ static glacier_hip_session *session_create_impl(glacier_hip_model *m,
     arg_bytes = std::max(arg_bytes, (size_t)r * sizeof(gk::ArgPartial) *
                                         std::max(0, gk::gemv_argmax_parts((int)c.vocab_size,
                                                                           (int)c.dim, (int)r,
-                                                                          head_D(s))));
+                                                                          head_D(s, (int)r))));
   A(&s->arg_scratch, arg_bytes);
   // GEMM split-K partial sums: the most any projection asks for at the row
   // counts past the GEMV (decode lanes up to 32, a full prompt chunk),
@@ -1892,7 +1895,7 @@ static glacier_hip_session *session_create_impl(glacier_hip_model *m,
     for (uint32_t rows : {(uint32_t)gk::kGemvMaxRows + 1, 24u, 32u, M})
       if (rows > (uint32_t)gk::kGemvMaxRows && rows <= M)
         for (const auto *w : ws)
-          for (int D : {1, 3}) {
+          for (int D : {gk::kPlanesQ8, gk::kPlanesSplit16}) {
             need = std::max(need, gk::gemm_splitk_floats((int)w->out_f, (int)rows, (int)w->in_f, D));
             // plane emission from the finishing pass needs the partial sums
             // even without a K split (decode lanes up to 32)

@@ -303,10 +303,11 @@ int glacier_hip_int4_gemv(glacier_hip_context *ctx, glacier_hip_int4_weight *wei
 /* glacier_hip_int4_gemv without any allocation. No counterpart in the
  * reference: for callers that cannot allocate device memory (code under HIP
  * graph capture, tight serving loops, harnesses that forbid hipMalloc). Its
- * activation planes and GEMM split-K partial sums live in one fixed 16 MiB
- * array per GPU (4 MiB of planes, 12 MiB of partial sums), held from the
+ * activation planes and GEMM split-K partial sums live in one fixed 17.5 MiB
+ * array per GPU (5.5 MiB of planes, 12 MiB of partial sums), held from the
  * library's load until the process ends; m is at most 64 rows and the planes
- * of m x in_f at most 4 MiB (SHAPE_MISMATCH otherwise, nothing launched).
+ * of m x in_f at most 4 MiB, f32 activations counted at three bytes an
+ * element (SHAPE_MISMATCH otherwise, nothing launched).
  * Same arithmetic as glacier_hip_int4_gemv (a smaller workspace may lower a
  * K split, which reorders only the f32 sum across splits). Every call on one
  * GPU shares that array: calls that overlap on a GPU (from several threads
@@ -322,7 +323,8 @@ int glacier_hip_int4_gemv_noalloc(glacier_hip_context *ctx, glacier_hip_int4_wei
  * int4_neon.c:453-486) and linearInt4WeightQ8Prepared (int4_matmul.zig:771):
  * the activation is converted once into device "digit planes" that several
  * projections with the same in_f can share. activation must be Q8 or F32
- * (F32 = three digit planes). act_dev must hold
+ * (F32 = three 7-bit digit planes up to 2 rows, an fp16 hi + lo pair per
+ * element above; planes belong to the m they were prepared for). act_dev must hold
  * glacier_hip_activation_bytes(m, in_f, activation) bytes. */
 uint64_t glacier_hip_activation_bytes(uint32_t m, uint32_t in_f, int activation);
 int glacier_hip_activation_prepare(glacier_hip_context *ctx, const void *x_dev, int x_dtype,
