@@ -2005,173 +2005,208 @@ hipError_t launch_attn_o(const AttnOArgs &a, hipStream_t st) {
 // q . k / sqrt(hd) over the row's positions 0 .. pos, then the weighted sum
 // of v), fp16 KV pages.
 //
-// Workgroup = the G query heads of one KV head (one wave each) x 16 query
-// rows; it walks the key pages 0 .. (last row's position) / 16, staging each
-// page's K rows and V (transposed) in LDS, double buffered, one barrier per
-// page, so the G waves share every K/V read. Per page and wave:
-//   * S^T = K . Q^T as one 16 x 16 tile (keys x rows) with f16 MFMAs; Q is
-//     split into f16 hi + lo parts (K is exact in f16), so the scores carry
-//     f32 accuracy like the decode kernel's;
-//   * online softmax per row (column of S^T: the 16 keys of row j sit in
-//     lanes (c, j), c = 0..3, four per lane), causal mask on the diagonal;
-//   * O += P . V with P split into f16 hi + lo (the tile's A operand is the
-//     lane's own P registers) and V^T from LDS; O (16 rows x hd, f32) stays
-//     in registers, rescaled by each row's exp(m_old - m_new).
-// The last blocks (longest key ranges) are scheduled first. PPT: 16-byte
-// K (and V) pieces each thread stages per page (16 * hd / 8 pieces over
-// 64 * G threads).
-template <int HD, int PPT>
-__global__ __launch_bounds__(64 * kMaxGroup) void attn_prefill_kernel(
+// Workgroup = the G query heads of one KV head x R tiles of 16 query rows, a
+// wave each (R = 8 / G, so small groups still share every K/V read among
+// about 8 waves). It walks the keys 32 (two pages) at a time, staged in LDS
+// double buffered with one barrier per 32 keys: K rows, and V transposed (4
+// keys x 4 dims per thread through byte permutes and 8-byte writes). Per 32
+// keys and wave:
+//   * S^T = K . Q^T as two 16 x 16 tiles (keys x rows) on f16 MFMAs with
+//     K = 32; Q is split into f16 hi + lo parts (K is exact in f16);
+//   * online softmax per row: column j of S^T lies in lanes (c, j), so the
+//     running maximum costs two cross-row exchanges, the sums stay per lane
+//     until the end, and p = 2^(s c - m c), c = log2(e) / sqrt(hd), is one fma
+//     and one exponential; keys are compared with the row's position only
+//     where the causal edge passes; O is rescaled only when some row's
+//     maximum grew;
+//   * O^T += V^T . P^T with P split into f16 hi + lo: the B operand is the
+//     lane's own P registers (V's slots are stored in that key order) and a
+//     lane's outputs belong to its own row j, so factors need no exchange.
+// Bound: matrix and vector issue, 32 MFMAs (about 530 cycles) and about 330
+// cycles of vector work per 32 keys x 16 rows x head, half of the time at 2048
+// rows of 28 / 4 heads of 128: 97 us. 285 us before, with 16 keys a barrier,
+// K = 16 MFMAs, O rescaled and row factors exchanged every 16 keys and V
+// transposed through 2-byte writes.
+// Order: workgroup b takes the b-th longest block, every second run of 256
+// reversed, so a CU's two workgroups are a long and a short one.
+// ---------------------------------------------------------------------------
+constexpr int kPfKeys = 32;
+template <int HD, int KPP>
+__global__ __launch_bounds__(64 * kMaxGroup, 4) void attn_prefill_kernel(
     const float *q, const __half *pool, const int32_t *ptab, int pos0, int T, int layer,
-    int num_layers, int Hq, int Hkv, float *out) {
-  typedef _Float16 h4 __attribute__((ext_vector_type(4)));
+    int num_layers, int Hq, int Hkv, int R, float *out) {
+  typedef _Float16 h8 __attribute__((ext_vector_type(8)));
   typedef float f4 __attribute__((ext_vector_type(4)));
-  constexpr int S = HD / 16;   // 16-wide steps over the head dim (scores)
-  constexpr int NT = HD / 16;  // 16-wide output tiles over the head dim
-  constexpr int KP = HD + 8;   // K row stride in halves (padded)
-  constexpr int VP = 16 + 4;   // V^T row stride in halves (padded)
-  constexpr int PIECES = 16 * HD / 8;  // 16-byte pieces of one page's K (or V)
-  __shared__ __align__(16) _Float16 ks[2][16 * KP];
+  constexpr int S = HD / 32;            // steps over the head dim (scores)
+  constexpr int NT = HD / 16;           // 16-wide output tiles over the head dim
+  constexpr int KP = HD + 8;            // K row stride in halves (padded)
+  constexpr int VP = kPfKeys + 8;       // V^T row stride in halves (padded)
+  constexpr int KPIECES = kPfKeys * HD / 8;      // 16-byte pieces of a stage's K
+  constexpr int VBLOCKS = kPfKeys / 4 * HD / 4;  // 4 keys x 4 dims of its V
+  __shared__ __align__(16) _Float16 ks[2][kPfKeys * KP];
   __shared__ __align__(16) _Float16 vt[2][HD * VP];
-  const int t = threadIdx.x, l = t & 63;
+  const int t = threadIdx.x, l = t & 63, nthr = (int)blockDim.x;
   const int wv = __builtin_amdgcn_readfirstlane(t >> 6);
   const int c = l >> 4, j = l & 15;
   const int G = Hq / Hkv;
-  const int nqb = (T + 15) / 16;
-  const int i0 = (nqb - 1 - (int)blockIdx.x) * 16;  // longest blocks first
-  const int h = blockIdx.y;
-  const int qh = h * G + wv;
+  const int BQ = 16 * R, nqb = (T + BQ - 1) / BQ;
+  // longest blocks first, every second run of 256 reversed
+  const int W = (int)gridDim.x, b = (int)blockIdx.x, run = b >> 8;
+  const int rank = run & 1 ? 256 * run + min(256, W - 256 * run) - 1 - (b & 255) : b;
+  const int h = rank % Hkv;
+  const int i0 = (nqb - 1 - rank / Hkv) * BQ + 16 * (wv / G);  // this wave's rows
+  const int last_row = min((nqb - rank / Hkv) * BQ, T) - 1;    // the workgroup's
+  const int qh = h * G + wv % G;
   const int kv_dim = Hkv * HD;
   const size_t lay = (size_t)num_layers;
-  const int last_pos = pos0 + min(i0 + 15, T - 1);
-  const int npages = last_pos / 16 + 1;
-  const float scale = 1.0f / sqrtf((float)HD);
+  const int last_pos = pos0 + last_row;
+  const int nst = last_pos / kPfKeys + 1;
+  const float cl2 = 1.44269504088896341f / sqrtf((float)HD);
 
-  // staging: thread t moves K and V pieces t + 64 G i (i < PPT) of a page;
-  // key positions past the last row's are zeroed (their page slots may hold
-  // anything, and a masked score still multiplies its V row)
-  const int nthr = (int)blockDim.x;
-  uint4 kreg[PPT], vreg[PPT];
-  auto fetch = [&](int kp) {
-    const size_t pbase = ((size_t)ptab[kp] * lay + layer) * 2;
+  // staging: this thread's K pieces t + nthr i and V block t; keys past the
+  // last row's read that row again (their scores are masked)
+  v4u kreg[KPP];
+  v2u vreg[4];
+  const int vkq = t % (kPfKeys / 4), vd = t / (kPfKeys / 4) * 4;  // key quad, first dim
+  // (the two pages' ids are scalar loads a stage ahead of the rows')
+  const auto page = [&](int i) { return ptab[min(i, last_pos >> 4)]; };
+  int pg0 = page(0), pg1 = page(1);
+  const auto fetch = [&](int st) {
+    const _Float16 *pool16 = (const _Float16 *)pool + (size_t)h * HD;
+    const _Float16 *p0 = pool16 + ((size_t)pg0 * lay + layer) * 32 * kv_dim;
+    const _Float16 *p1 = pool16 + ((size_t)pg1 * lay + layer) * 32 * kv_dim;
+    const int last = last_pos - st * kPfKeys;  // of this stage's keys
+    const auto row = [&](int key) {
+      const int k = min(key, last);
+      return (k & 16 ? p1 : p0) + (k & 15) * kv_dim;
+    };
 #pragma unroll
-    for (int i = 0; i < PPT; ++i) {
-      const int pc = t + nthr * i, skey = pc / (HD / 8), spc = pc % (HD / 8);
-      kreg[i] = vreg[i] = make_uint4(0, 0, 0, 0);
-      if (pc < PIECES && 16 * kp + skey <= last_pos) {
-        const size_t off = (pbase * 16 + skey) * kv_dim + (size_t)h * HD + 8 * spc;
-        kreg[i] = *(const uint4 *)(pool + off);
-        vreg[i] = *(const uint4 *)(pool + off + 16 * (size_t)kv_dim);
+    for (int i = 0; i < KPP; ++i) {
+      const int pc = min(t + nthr * i, KPIECES - 1);
+      kreg[i] = *(const v4u *)(row(pc / (HD / 8)) + 8 * (pc % (HD / 8)));
+    }
+    if (t < VBLOCKS) {
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        vreg[k] = *(const v2u *)(row(4 * vkq + k) + 16 * kv_dim + vd);
+    }
+    pg0 = page(2 * st + 2);
+    pg1 = page(2 * st + 3);
+  };
+  const auto stage = [&](int bi) {
+#pragma unroll
+    for (int i = 0; i < KPP; ++i) {
+      const int pc = min(t + nthr * i, KPIECES - 1);
+      *(v4u *)&ks[bi][pc / (HD / 8) * KP + 8 * (pc % (HD / 8))] = kreg[i];
+    }
+    if (t < VBLOCKS) {
+      // slot of key 16 T + 4 c + r: 8 c + 4 T + r, the order of P's registers
+      _Float16 *d = &vt[bi][vd * VP + 8 * (vkq & 3) + 4 * (vkq >> 2)];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const uint32_t sel = e & 1 ? 0x07060302u : 0x05040100u;
+        v2u w;
+        w.x = __builtin_amdgcn_perm(vreg[1][e >> 1], vreg[0][e >> 1], sel);
+        w.y = __builtin_amdgcn_perm(vreg[3][e >> 1], vreg[2][e >> 1], sel);
+        *(v2u *)(d + e * VP) = w;
       }
     }
   };
-  auto stage = [&](int b) {
-#pragma unroll
-    for (int i = 0; i < PPT; ++i) {
-      const int pc = t + nthr * i, skey = pc / (HD / 8), spc = pc % (HD / 8);
-      if (pc >= PIECES) continue;
-      *(uint4 *)&ks[b][skey * KP + 8 * spc] = kreg[i];
-      const _Float16 *vh = (const _Float16 *)&vreg[i];
-#pragma unroll
-      for (int e = 0; e < 8; ++e) vt[b][(8 * spc + e) * VP + skey] = vh[e];
-    }
-  };
   fetch(0);
-  stage(0);
 
-  // Q^T as the B operand: lane (c, j) = row i0 + j, dims 16 st + 4c .. + 3
-  h4 qhi[S], qlo[S];
+  // Q^T as the B operand: lane (c, j) = row i0 + j, dims 32 st + 8 c .. + 7
+  h8 qhi[S], qlo[S];
   {
     const float *qrow = q + ((size_t)min(i0 + j, T - 1) * Hq + qh) * HD;
 #pragma unroll
     for (int st = 0; st < S; ++st) {
-      const float4 qv = *(const float4 *)(qrow + 16 * st + 4 * c);
-      const float qa[4] = {qv.x, qv.y, qv.z, qv.w};
+      const float4 qa = *(const float4 *)(qrow + 32 * st + 8 * c);
+      const float4 qb = *(const float4 *)(qrow + 32 * st + 8 * c + 4);
+      const float qv[8] = {qa.x, qa.y, qa.z, qa.w, qb.x, qb.y, qb.z, qb.w};
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const _Float16 hv = (_Float16)qa[e];
+      for (int e = 0; e < 8; ++e) {
+        const _Float16 hv = (_Float16)qv[e];
         qhi[st][e] = hv;
-        qlo[st][e] = (_Float16)(qa[e] - (float)hv);
+        qlo[st][e] = (_Float16)(qv[e] - (float)hv);
       }
     }
   }
-  const int qpos = pos0 + i0 + j;  // position of this lane's score column
+  stage(0);
+  const int qpos = pos0 + i0 + j;  // position of this lane's row
   f4 o[NT];
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt) o[nt] = f4{0.0f, 0.0f, 0.0f, 0.0f};
   float mx = -INFINITY, sum = 0.0f;
   __syncthreads();
 
-  for (int kp = 0; kp < npages; ++kp) {
-    const int b = kp & 1;
-    if (kp + 1 < npages) fetch(kp + 1);  // next page in flight
-    // scores S^T[key 4c + r][row j]; every K fragment is read from LDS
-    // before the first MFMA (one LDS round trip a page, not one a step)
-    h4 kf[S];
+  for (int st = 0; st < nst; ++st) {
+    const int bi = st & 1;
+    if (st + 1 < nst) fetch(st + 1);  // the next keys in flight
+    f4 acc[2];
 #pragma unroll
-    for (int st = 0; st < S; ++st) kf[st] = *(const h4 *)&ks[b][j * KP + 16 * st + 4 * c];
-    __builtin_amdgcn_sched_barrier(0);  // (the scheduler would sink them again)
-    f4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int tt = 0; tt < 2; ++tt) {
+      acc[tt] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+      h8 kf[S];
 #pragma unroll
-    for (int st = 0; st < S; ++st) {
-      acc = __builtin_amdgcn_mfma_f32_16x16x16f16(kf[st], qhi[st], acc, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_f32_16x16x16f16(kf[st], qlo[st], acc, 0, 0, 0);
+      for (int s2 = 0; s2 < S; ++s2)
+        kf[s2] = *(const h8 *)&ks[bi][(16 * tt + j) * KP + 32 * s2 + 8 * c];
+#pragma unroll
+      for (int s2 = 0; s2 < S; ++s2)  // (the small terms first: fewer roundings at full size)
+        acc[tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[s2], qlo[s2], acc[tt], 0, 0, 0);
+#pragma unroll
+      for (int s2 = 0; s2 < S; ++s2)
+        acc[tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[s2], qhi[s2], acc[tt], 0, 0, 0);
     }
-    // the V fragments do not depend on the softmax: requested before it
-    __builtin_amdgcn_sched_barrier(0);
-    h4 vf[NT];
+    float sv[8], pm = -INFINITY;
 #pragma unroll
-    for (int nt = 0; nt < NT; ++nt) vf[nt] = *(const h4 *)&vt[b][(16 * nt + j) * VP + 4 * c];
-    __builtin_amdgcn_sched_barrier(0);
-    float sv[4], pm = -INFINITY;
+    for (int e = 0; e < 8; ++e) sv[e] = acc[e >> 2][e & 3];
+    if (st * kPfKeys + kPfKeys - 1 > pos0 + i0) {  // the causal edge passes here (uniform)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int kpos = 16 * kp + 4 * c + r;
-      sv[r] = kpos <= qpos ? acc[r] * scale : -INFINITY;
-      pm = fmaxf(pm, sv[r]);
+      for (int e = 0; e < 8; ++e)
+        if (st * kPfKeys + 16 * (e >> 2) + 4 * c + (e & 3) > qpos) sv[e] = -INFINITY;
     }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) pm = fmaxf(pm, sv[e]);
     pm = xor32_max(xor16_max(pm));
-    const float mnew = fmaxf(mx, pm);  // finite: key 0 is in every row's range
-    const float alpha = expf(mx - mnew);
-    h4 phi, plo;
-    float ps = 0.0f;
+    // (a row past the workgroup's keys keeps its finite maximum: key 0 is in
+    // every row's range)
+    if (__any(pm > mx)) {
+      const float mnew = fmaxf(mx, pm);
+      const float alpha = __builtin_amdgcn_exp2f((mx - mnew) * cl2);
+      sum *= alpha;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const float pv = expf(sv[r] - mnew);
-      ps += pv;
-      const _Float16 hv = (_Float16)pv;
-      phi[r] = hv;
-      plo[r] = (_Float16)(pv - (float)hv);
+      for (int nt = 0; nt < NT; ++nt) o[nt] *= alpha;
+      mx = mnew;
     }
-    ps = xor32_add(xor16_add(ps));
-    sum = sum * alpha + ps;
-    mx = mnew;
-    // O rows are rows 4c + r: their factors live in lanes 4c + r
-    float ar[4];
+    const float m2 = mx * cl2;
+    h8 phi, plo;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) ar[r] = __shfl(alpha, 4 * c + r);
+    for (int e = 0; e < 8; ++e) {
+      const float pv = __builtin_amdgcn_exp2f(fmaf(sv[e], cl2, -m2));
+      sum += pv;
+      const _Float16 hv = (_Float16)pv;
+      phi[e] = hv;
+      plo[e] = (_Float16)(pv - (float)hv);
+    }
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) o[nt][r] *= ar[r];
-      o[nt] = __builtin_amdgcn_mfma_f32_16x16x16f16(phi, vf[nt], o[nt], 0, 0, 0);
-      o[nt] = __builtin_amdgcn_mfma_f32_16x16x16f16(plo, vf[nt], o[nt], 0, 0, 0);
+      const h8 vf = *(const h8 *)&vt[bi][(16 * nt + j) * VP + 8 * c];
+      o[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf, phi, o[nt], 0, 0, 0);
+      o[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf, plo, o[nt], 0, 0, 0);
     }
-    // publish the next page (the other buffer was last read before the
+    // publish the next keys (the other buffer was last read before the
     // previous barrier)
-    if (kp + 1 < npages) stage(b ^ 1);
+    if (st + 1 < nst) stage(bi ^ 1);
     __syncthreads();
   }
-  // lane (c, j): O[row 4c + r][dim 16 nt + j]
+  // lane (c, j): O[row j][dims 16 nt + 4 c .. + 3]
+  sum = xor32_add(xor16_add(sum));
+  if (i0 + j < T) {
+    float *orow = out + ((size_t)(i0 + j) * Hq + qh) * HD;
 #pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const int row = i0 + 4 * c + r;
-    const float lr = __shfl(sum, 4 * c + r);
-    if (row < T) {
-      float *orow = out + ((size_t)row * Hq + qh) * HD;
-#pragma unroll
-      for (int nt = 0; nt < NT; ++nt) orow[16 * nt + j] = o[nt][r] / lr;
-    }
+    for (int nt = 0; nt < NT; ++nt)
+      *(f4 *)(orow + 16 * nt + 4 * c) =
+          f4{o[nt][0] / sum, o[nt][1] / sum, o[nt][2] / sum, o[nt][3] / sum};
   }
 }
 
@@ -2184,16 +2219,16 @@ hipError_t launch_attention_prefill(const float *q, const void *kv_pool, const i
     return hipErrorInvalidValue;
   const int G = num_heads / num_kv_heads;
   if (head_dim != 64 && head_dim != 128) return hipErrorInvalidValue;
-  const dim3 grid((T + 15) / 16, num_kv_heads), block(64 * G);
+  const int R = kMaxGroup / G;  // 320 to 512 threads
+  const dim3 grid((T + 16 * R - 1) / (16 * R) * num_kv_heads), block(64 * G * R);
   const int32_t *ptab = page_table + (size_t)lane * max_pages;
   const __half *pool = (const __half *)kv_pool;
-  const int ppt = (16 * head_dim / 8 + 64 * G - 1) / (64 * G);
-#define GK_PF(HD, P)                                                                              hipLaunchKernelGGL((attn_prefill_kernel<HD, P>), grid, block, 0, st, q, pool, ptab, pos0, T,                      layer, num_layers, num_heads, num_kv_heads, out)
-  if (head_dim == 64) {
-    if (ppt <= 1) GK_PF(64, 1); else GK_PF(64, 2);
-  } else {
-    if (ppt <= 1) GK_PF(128, 1); else if (ppt == 2) GK_PF(128, 2); else GK_PF(128, 4);
-  }
+#define GK_PF(HD, P)                                                                             \
+  hipLaunchKernelGGL((attn_prefill_kernel<HD, P>), grid, block, 0, st, q, pool, ptab, pos0, T,   \
+                     layer, num_layers, num_heads, num_kv_heads, R, out)
+  if (head_dim == 64) GK_PF(64, 1);
+  else if (block.x == 64 * kMaxGroup) GK_PF(128, 1);
+  else GK_PF(128, 2);
 #undef GK_PF
   return hipGetLastError();
 }

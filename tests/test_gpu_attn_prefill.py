@@ -1,0 +1,68 @@
+"""Edges of the prompt-chunk attention kernel (glacier_hip_paged_attention_prefill)
+against 64-bit sums: chunks around its 16-row wave tiles and 32-key stages,
+every group size from 1 to 8 query heads per KV head (1 to 8 waves, row tiles
+filled up to 8), both head widths, chunks that start mid-page, scattered
+pages whose unused slots hold NaN, and one row that dominates its softmax.
+
+Bar: 2e-6 of the largest output. Scores carry f32 accumulation rounding
+(|q . k| up to ~60 here: 2^-19 absolute, 3e-7 in the exponent after the
+1 / sqrt(hd) factor), outputs the fp16 hi + lo split of the weights (2^-22).
+"""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+LAYERS, LAYER = 3, 1
+
+
+def _case(gh, gctx, Hq, Hkv, hd, pos0, T, seed):
+    import torch
+
+    g = torch.Generator().manual_seed(seed)
+    end = pos0 + T
+    npages = -(-end // 16)
+    perm = torch.randperm(npages + 2, generator=g)
+    pool = torch.full((npages + 2, LAYERS, 2, 16, Hkv * hd), float("nan"), dtype=torch.float16)
+    kv = torch.randn((2, end, Hkv * hd), generator=g).half()
+    for p in range(end):
+        pool[perm[p // 16], LAYER, :, p % 16] = kv[:, p]
+    q = 1.5 * torch.randn((T, Hq, hd), generator=g)
+    q[T // 2] *= 4.0
+    table = perm[:npages].to(torch.int32)
+    qd, pd, td = q.reshape(T, -1).cuda(), pool.cuda(), table.cuda()
+    out = torch.full((T + 1, Hq * hd), 5.0, device="cuda")
+    torch.cuda.synchronize()
+    gh.check(gh.lib().glacier_hip_paged_attention_prefill(
+        gctx.h, qd.data_ptr(), pd.data_ptr(), td.data_ptr(), npages, pos0, T, LAYER, LAYERS, Hq, Hkv,
+        hd, out.data_ptr(), None), "attention_prefill", gctx.h)
+    gctx.sync()
+    got = out.cpu().numpy()
+    assert np.all(got[T] == 5.0)
+    kvd = kv.double().view(2, end, Hkv, hd)
+    want = np.empty((T, Hq, hd))
+    mask = torch.arange(end)[None, :] > (pos0 + torch.arange(T))[:, None]
+    for h in range(Hq):
+        kh = h // (Hq // Hkv)
+        sc = (q[:, h].double() @ kvd[0, :, kh].T) / np.sqrt(hd)
+        want[:, h] = (torch.softmax(sc.masked_fill(mask, -np.inf), -1) @ kvd[1, :, kh]).numpy()
+    err = np.max(np.abs(got[:T].reshape(T, Hq, hd) - want)) / np.max(np.abs(want))
+    assert err < 2e-6, err
+
+
+@pytest.mark.parametrize("T", [1, 15, 16, 17, 31, 33, 64, 97])
+@pytest.mark.parametrize("pos0", [0, 1, 15, 16, 33, 47])
+@pytest.mark.parametrize("hd", [64, 128])
+def test_chunk_edges(gh, gctx, T, pos0, hd):
+    _case(gh, gctx, 14, 2, hd, pos0, T, 100 * T + pos0)
+
+
+@pytest.mark.parametrize("G", [1, 2, 3, 4, 5, 6, 8])
+@pytest.mark.parametrize("hd", [64, 128])
+def test_group_sizes(gh, gctx, G, hd):
+    _case(gh, gctx, 2 * G, 2, hd, 21, 150, G)
+
+
+def test_more_workgroups_than_a_run(gh, gctx):
+    """Over 512 workgroups (three runs of 256 in the block order)."""
+    _case(gh, gctx, 40, 8, 64, 5, 1100, 7)
