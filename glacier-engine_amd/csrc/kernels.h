@@ -220,15 +220,6 @@ hipError_t launch_attention(const float *q, const void *kv_pool, int kv_f16,
                             float *scratch, float *out, hipStream_t st,
                             PlanesDst emit = PlanesDst{nullptr, nullptr, 1});
 
-// fp16-KV attention with an explicit launch shape: wp positions per wave,
-// nw waves per workgroup (tuning; launch_attention picks the shape).
-hipError_t launch_attention_f16(const float *q, const void *kv_pool, const int32_t *page_table,
-                                int max_pages, const int32_t *lane_of_row, const int32_t *ctx_len,
-                                int M, int layer, int num_layers, int num_heads, int num_kv_heads,
-                                int head_dim, int max_ctx, float *scratch, float *out,
-                                hipStream_t st, int wp, int nw,
-                                PlanesDst emit = PlanesDst{nullptr, nullptr, 1});
-
 // Batch-1 decode with fp16 KV: attention fused with the O projection.
 // Workgroup (row-block group bg, KV head h) computes the attention of the
 // G = Hq / Hkv query heads of KV head h over row 0's whole context, quantises

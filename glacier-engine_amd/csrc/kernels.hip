@@ -853,8 +853,10 @@ hipError_t launch_gather_rows(const float *table, const int32_t *ids, int M, int
 // ---------------------------------------------------------------------------
 // grid (chunks, kv heads, rows). A workgroup serves the G = Hq / Hkv query
 // heads that share one KV head over one context chunk. HD/8 threads cooperate
-// on a position (one 16-byte fp16 load each), so K and V rows are read fully
-// coalesced straight from the lane's pages. One chunk: the output is written
+// on a position (two 16-byte loads each), so K and V rows are read fully
+// coalesced straight from the lane's pages. f32 KV, for prompt chunks (a row
+// per workgroup plane) and contexts past the work list's records; decode steps
+// run the work list below. One chunk: the output is written
 // directly with the weights normalised first (forward.zig:515-528); several
 // chunks: (max, sum, unnormalised output) records are merged by the combine
 // kernel with the usual log-sum-exp rescaling.
@@ -888,24 +890,16 @@ size_t attention_scratch_floats(int max_rows, int num_heads, int num_kv_heads, i
   return most;
 }
 
-template <int HD, int F16>
-static __device__ __forceinline__ void load8(const void *pool, size_t idx, float *v) {
-  if (F16) {
-    const uint4 raw = *(const uint4 *)((const __half *)pool + idx);
-    const __half *hp = (const __half *)&raw;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) v[e] = __half2float(hp[e]);
-  } else {
-    const float4 r0 = *(const float4 *)((const float *)pool + idx);
-    const float4 r1 = *(const float4 *)((const float *)pool + idx + 4);
-    v[0] = r0.x; v[1] = r0.y; v[2] = r0.z; v[3] = r0.w;
-    v[4] = r1.x; v[5] = r1.y; v[6] = r1.z; v[7] = r1.w;
-  }
+static __device__ __forceinline__ void load8(const float *p, float *v) {
+  const float4 r0 = *(const float4 *)p;
+  const float4 r1 = *(const float4 *)(p + 4);
+  v[0] = r0.x; v[1] = r0.y; v[2] = r0.z; v[3] = r0.w;
+  v[4] = r1.x; v[5] = r1.y; v[6] = r1.z; v[7] = r1.w;
 }
 
-template <int HD, int F16, int HPW>
+template <int HD>
 __global__ __launch_bounds__(256) void attn_decode_kernel(
-    const float *q, const void *kv_pool, const int32_t *page_table, int max_pages,
+    const float *q, const float *kv_pool, const int32_t *page_table, int max_pages,
     const int32_t *lane_of_row, const int32_t *ctx_len, int layer, int num_layers, int Hq,
     int Hkv, int chunk, int n_chunks_max, int max_ctx, float *scratch, float *out,
     PlanesDst pd) {
@@ -913,12 +907,7 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(
   constexpr int PPP = 256 / TPP;     // positions per pass
   constexpr int PPW = 64 / TPP;      // positions per wave
   const int ch = blockIdx.x, m = blockIdx.z, t = threadIdx.x;
-  // HPW == 1: one query head per workgroup (blockIdx.y = query head);
-  // otherwise all G query heads of one KV head (blockIdx.y = KV head).
-  const int Gfull = Hq / Hkv;
-  const int h = HPW == 1 ? (int)blockIdx.y / Gfull : (int)blockIdx.y;
-  const int qh0 = HPW == 1 ? (int)blockIdx.y : h * Gfull;
-  const int G = HPW == 1 ? 1 : Gfull;
+  const int G = Hq / Hkv, h = blockIdx.y, qh0 = h * G;
   const int ctx = min(ctx_len[m], max_ctx);
   const int j0 = ch * chunk;
   if (j0 >= ctx) return;
@@ -926,10 +915,10 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(
   const int nch = (ctx + chunk - 1) / chunk;
   const int kv_dim = Hkv * HD;
   const int lane_id = lane_of_row[m];
-  __shared__ float sq[HPW][HD];
-  __shared__ float ss[HPW][kMaxChunk];
-  __shared__ float red[4][HPW][HD];
-  __shared__ float smax[HPW], ssum[HPW];
+  __shared__ float sq[kMaxGroup][HD];
+  __shared__ float ss[kMaxGroup][kMaxChunk];
+  __shared__ float red[4][kMaxGroup][HD];
+  __shared__ float smax[kMaxGroup], ssum[kMaxGroup];
   __shared__ int spage[kMaxChunk / 16];
   for (int i = t; i < G * HD; i += 256)
     sq[i / HD][i % HD] = q[(size_t)m * Hq * HD + (size_t)qh0 * HD + i];
@@ -941,60 +930,10 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(
   const float scale = 1.0f / sqrtf((float)HD);
   const size_t lay = (size_t)num_layers;
   // ---- scores ----
-  if constexpr (F16 && HPW == kMaxGroup) {
-    // fp16 KV: S[head][pos] = q . k on v_mfma_f32_16x16x16_f16, one 16-position
-    // tile (one page) per MFMA column block, query heads as MFMA rows. q is
-    // split into fp16 hi + lo parts (q = hi + lo to ~2^-22 relative); the
-    // fp16 x fp16 products are exact in the f32 accumulator, so the score is
-    // the f32 dot product up to summation order. Lane (c, j) loads 16-byte
-    // pieces 4*tt + c of position j's K row, which fixes the dims of k-chunk c
-    // in step s: 8 * (4 * (s / 2) + c) + 4 * (s % 2) + 0..3.
-    typedef _Float16 h4 __attribute__((ext_vector_type(4)));
-    typedef float f4 __attribute__((ext_vector_type(4)));
-    constexpr int S = HD / 16;
-    const int wv = t >> 6, l = t & 63, c = l >> 4, jr = l & 15;
-    h4 qhi[S], qlo[S];
+  {
+    float qf[kMaxGroup][8];
 #pragma unroll
-    for (int st = 0; st < S; ++st) {
-      const int base = 8 * (4 * (st >> 1) + c) + 4 * (st & 1);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const float v = jr < G ? sq[jr][base + e] : 0.0f;
-        const _Float16 hv = (_Float16)v;
-        qhi[st][e] = hv;
-        qlo[st][e] = (_Float16)(v - (float)hv);
-      }
-    }
-    for (int T = wv; T * 16 < n; T += 4) {
-      const int pl = T * 16 + jr;  // position within the chunk; page = spage[T]
-      const bool valid = pl < n;
-      const __half *krow = (const __half *)kv_pool +
-                           ((((size_t)spage[T] * lay + layer) * 2 + 0) * 16 + jr) * kv_dim +
-                           (size_t)h * HD;
-      uint4 kr[HD / 32];
-#pragma unroll
-      for (int tt = 0; tt < HD / 32; ++tt)
-        kr[tt] = valid ? *(const uint4 *)(krow + 8 * (4 * tt + c)) : make_uint4(0, 0, 0, 0);
-      f4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-      for (int st = 0; st < S; ++st) {
-        const uint4 w = kr[st >> 1];
-        const uint2 bw = (st & 1) ? make_uint2(w.z, w.w) : make_uint2(w.x, w.y);
-        h4 b;
-        __builtin_memcpy(&b, &bw, 8);
-        acc = __builtin_amdgcn_mfma_f32_16x16x16f16(qhi[st], b, acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_16x16x16f16(qlo[st], b, acc, 0, 0, 0);
-      }
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int head = 4 * c + r;
-        if (head < G && valid) ss[head][pl] = acc[r] * scale;
-      }
-    }
-  } else {
-    float qf[HPW][8];
-#pragma unroll
-    for (int g = 0; g < HPW; ++g)
+    for (int g = 0; g < kMaxGroup; ++g)
 #pragma unroll
       for (int e = 0; e < 8; ++e) qf[g][e] = g < G ? sq[g][sub * 8 + e] : 0.0f;
     constexpr int B = 8;  // rows in flight per thread
@@ -1008,7 +947,7 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(
           const size_t idx =
               ((((size_t)spage[i >> 4] * lay + layer) * 2 + 0) * 16 + (j & 15)) * kv_dim +
               (size_t)h * HD + sub * 8;
-          load8<HD, F16>(kv_pool, idx, kv[b]);
+          load8(kv_pool + idx, kv[b]);
         }
       }
 #pragma unroll
@@ -1016,7 +955,7 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(
         const int i = i0 + b * PPP;
         if (i >= n) break;
 #pragma unroll
-        for (int g = 0; g < HPW; ++g) {
+        for (int g = 0; g < kMaxGroup; ++g) {
           if (g >= G) break;
           float d = 0.0f;
 #pragma unroll
@@ -1055,9 +994,9 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(
   }
   __syncthreads();
   // ---- weighted V ----
-  float acc[HPW][8];
+  float acc[kMaxGroup][8];
 #pragma unroll
-  for (int g = 0; g < HPW; ++g)
+  for (int g = 0; g < kMaxGroup; ++g)
 #pragma unroll
     for (int e = 0; e < 8; ++e) acc[g][e] = 0.0f;
   {
@@ -1072,7 +1011,7 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(
           const size_t idx =
               ((((size_t)spage[i >> 4] * lay + layer) * 2 + 1) * 16 + (j & 15)) * kv_dim +
               (size_t)h * HD + sub * 8;
-          load8<HD, F16>(kv_pool, idx, v[b]);
+          load8(kv_pool + idx, v[b]);
         }
       }
 #pragma unroll
@@ -1080,7 +1019,7 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(
         const int i = i0 + b * PPP;
         if (i >= n) break;
 #pragma unroll
-        for (int g = 0; g < HPW; ++g) {
+        for (int g = 0; g < kMaxGroup; ++g) {
           if (g >= G) break;
           const float w = ss[g][i];
 #pragma unroll
@@ -1091,7 +1030,7 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(
   }
   // reduce over the positions of a wave (lanes sub + TPP * k), then over waves
 #pragma unroll
-  for (int g = 0; g < HPW; ++g) {
+  for (int g = 0; g < kMaxGroup; ++g) {
     if (g >= G) break;
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
@@ -1104,7 +1043,7 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(
   const int w = t >> 6, l = t & 63;
   if (l < TPP) {
 #pragma unroll
-    for (int g = 0; g < HPW; ++g) {
+    for (int g = 0; g < kMaxGroup; ++g) {
       if (g >= G) break;
 #pragma unroll
       for (int e = 0; e < 8; ++e) red[w][g][l * 8 + e] = acc[g][e];
@@ -1131,7 +1070,7 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// fp16-KV streaming attention. The work list is every (row, KV head, chunk
+// Streaming decode attention (fp16 or f32 KV). The work list is every (row, KV head, chunk
 // of CH = NW * NT * 16 positions) with each row's chunks counted from its own
 // context length, rows in order; workgroup b takes items b, b + grid, ...,
 // so no chunk past a row's context is ever launched for it. A wave owns NT
@@ -1391,7 +1330,13 @@ static __device__ __forceinline__ void attn_f16_item(const float *qrow, const __
 // Every load is unconditional from an in-range address (as there). q is
 // staged in LDS (qs, kMaxGroup * HD floats) by the whole workgroup and read
 // a float4 per step: f32 K and V rows take twice the registers of fp16 ones.
-template <int HD, int NT, int NW, class Hook = AttnNoHook>
+//
+// kExact: the products on v_mfma_f32_16x16x4f32 on the f32 values themselves
+// (any f32 range, every product rounded once into the sum): the list kernel's
+// form, whose waves hold one page each and wait for memory, not for MFMAs.
+// There a step's four k-chunks are the lanes' own elements (K, q: element e
+// of their quarters; P, V: positions 4 c + r).
+template <int HD, int NT, int NW, bool kExact, class Hook = AttnNoHook>
 static __device__ __forceinline__ void attn_f32_item(const float *qrow, const float *pool,
                                                      const int32_t *ptab, int n, int layer,
                                                      size_t lay, int kv_dim, int h, int G,
@@ -1465,32 +1410,42 @@ static __device__ __forceinline__ void attn_f32_item(const float *qrow, const fl
 #pragma unroll
     for (int T = 0; T < NT; ++T) {
       f4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+      f4 part[8] = {acc, acc, acc, acc, acc, acc, acc, acc};  // kExact: short sums, few roundings in each
 #pragma unroll
       for (int i = 0; i < QD / 4; ++i) {
         const float4 qv = *(const float4 *)(qr + 4 * i);
         const float qa[4] = {qon ? qv.x : 0.0f, qon ? qv.y : 0.0f, qon ? qv.z : 0.0f,
                              qon ? qv.w : 0.0f};
         const float ka[4] = {kr[T][i].x, kr[T][i].y, kr[T][i].z, kr[T][i].w};
-        h4 kh, kl, qh, ql;
-        split_f16(ka, kh, kl);
-        split_f16(qa, qh, ql);
-        acc = __builtin_amdgcn_mfma_f32_16x16x16f16(kh, qh, acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_16x16x16f16(kh, ql, acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_16x16x16f16(kl, qh, acc, 0, 0, 0);
+        if constexpr (kExact) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            part[(4 * i + e) & 7] = __builtin_amdgcn_mfma_f32_16x16x4f32(ka[e], qa[e], part[(4 * i + e) & 7], 0, 0, 0);
+        } else {
+          h4 kh, kl, qh, ql;
+          split_f16(ka, kh, kl);
+          split_f16(qa, qh, ql);
+          acc = __builtin_amdgcn_mfma_f32_16x16x16f16(kh, qh, acc, 0, 0, 0);
+          acc = __builtin_amdgcn_mfma_f32_16x16x16f16(kh, ql, acc, 0, 0, 0);
+          acc = __builtin_amdgcn_mfma_f32_16x16x16f16(kl, qh, acc, 0, 0, 0);
+        }
       }
+      if constexpr (kExact)
+        acc = ((part[0] + part[1]) + (part[2] + part[3])) + ((part[4] + part[5]) + (part[6] + part[7]));
 #pragma unroll
       for (int rr = 0; rr < 4; ++rr) {
-        const float v = acc[rr] * scale;
-        sc[T][rr] = 16 * T + 4 * c + rr < wn ? v : -INFINITY;
+        sc[T][rr] = 16 * T + 4 * c + rr < wn ? (kExact ? acc[rr] : acc[rr] * scale) : -INFINITY;
         mx = fmaxf(mx, sc[T][rr]);
       }
     }
     mx = xor32_max(xor16_max(mx));
+    if constexpr (kExact) mx *= scale;
 #pragma unroll
     for (int T = 0; T < NT; ++T)
 #pragma unroll
       for (int rr = 0; rr < 4; ++rr) {
-        const float p = expf(sc[T][rr] - mx);
+        // (kExact: the score is not rounded before the maximum is taken off)
+        const float p = expf(kExact ? fmaf(sc[T][rr], scale, -mx) : sc[T][rr] - mx);
         sc[T][rr] = p;
         sum += p;
       }
@@ -1512,11 +1467,24 @@ static __device__ __forceinline__ void attn_f32_item(const float *qrow, const fl
 #pragma unroll
       for (int e = 0; e < DPL; ++e) {
         const float va[4] = {v0[e], v1[e], v2[e], v3[e]};
-        h4 vh, vl;
-        split_f16(va, vh, vl);
-        o[e] = __builtin_amdgcn_mfma_f32_16x16x16f16(ph, vh, o[e], 0, 0, 0);
-        o[e] = __builtin_amdgcn_mfma_f32_16x16x16f16(ph, vl, o[e], 0, 0, 0);
-        o[e] = __builtin_amdgcn_mfma_f32_16x16x16f16(pl, vh, o[e], 0, 0, 0);
+        if constexpr (kExact) {
+          // (two sums of half the positions where the registers allow it)
+          f4 odd = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+          for (int rr = 0; rr < 4; ++rr) {
+            if (NW < 16 && rr >= 2)
+              odd = __builtin_amdgcn_mfma_f32_16x16x4f32(pa[rr], va[rr], odd, 0, 0, 0);
+            else
+              o[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(pa[rr], va[rr], o[e], 0, 0, 0);
+          }
+          if constexpr (NW < 16) o[e] += odd;
+        } else {
+          h4 vh, vl;
+          split_f16(va, vh, vl);
+          o[e] = __builtin_amdgcn_mfma_f32_16x16x16f16(ph, vh, o[e], 0, 0, 0);
+          o[e] = __builtin_amdgcn_mfma_f32_16x16x16f16(ph, vl, o[e], 0, 0, 0);
+          o[e] = __builtin_amdgcn_mfma_f32_16x16x16f16(pl, vh, o[e], 0, 0, 0);
+        }
       }
     }
   }
@@ -1524,7 +1492,7 @@ static __device__ __forceinline__ void attn_f32_item(const float *qrow, const fl
 }
 
 // ---------------------------------------------------------------------------
-// fp16-KV streaming attention. The work list is every (row, KV head, chunk
+// Streaming decode attention (fp16 or f32 KV). The work list is every (row, KV head, chunk
 // of CH = NW * NT * 16 positions) with each row's chunks counted from its own
 // context length, rows in order; workgroup b takes items b, b + grid, ...,
 // so no chunk past a row's context is ever launched for it. A wave owns NT
@@ -1547,10 +1515,14 @@ static __device__ __forceinline__ void attn_f32_item(const float *qrow, const fl
 // whose context is one chunk writes its output normalised once by the sum
 // (forward.zig:515-528); otherwise every chunk writes a (max, sum, output)
 // record per query head for the combine kernel.
+// f32 pages run the same list with attn_f32_item, one page per wave and f32
+// MFMAs; bound by the latency of the page walk and the loads behind it. 6 lanes
+// of 14 / 2 heads of 64 at contexts 37 to 4096: 18.4 us with attn_decode_kernel
+// (scalar dots, 512-position chunks) -> 8.9.
 // ---------------------------------------------------------------------------
-template <int HD, int NT, int NW>
-__global__ __launch_bounds__(64 * NW) void attn_f16_kernel(
-    const float *q, const __half *pool, const int32_t *page_table, int max_pages,
+template <int HD, int NT, int NW, bool KV32>
+__global__ __launch_bounds__(64 * NW) void attn_list_kernel(
+    const float *q, const void *pool, const int32_t *page_table, int max_pages,
     const int32_t *lane_of_row, const int32_t *ctx_len, int M, int layer, int num_layers, int Hq,
     int Hkv, int n_chunks_max, int max_ctx, float *scratch, float *out, PlanesDst pd) {
   constexpr int WP = 16 * NT;   // positions per wave
@@ -1560,6 +1532,7 @@ __global__ __launch_bounds__(64 * NW) void attn_f16_kernel(
   const int G = Hq / Hkv;
   const int kv_dim = Hkv * HD;
   __shared__ AttnF16Lds<HD, NW> s;
+  __shared__ __align__(16) float qs[KV32 ? kMaxGroup * HD : 4];  // f32 items' q
 
   // the work list (every wave holds it; lane r describes row r, M <= 64)
   const int cl = l < M ? min(ctx_len[l], max_ctx) : 0;
@@ -1585,9 +1558,14 @@ __global__ __launch_bounds__(64 * NW) void attn_f16_kernel(
     const int h = r / nch, ch = r - h * nch;
     const int qh0 = h * G;
     const int j0 = ch * CH;
-    attn_f16_item<HD, NT, NW>(q + ((size_t)m * Hq + qh0) * HD, pool,
-                              page_table + (size_t)lane * max_pages + j0 / 16, min(CH, ctx - j0),
-                              layer, (size_t)num_layers, kv_dim, h, G, s);
+    const float *qrow = q + ((size_t)m * Hq + qh0) * HD;
+    const int32_t *ptab = page_table + (size_t)lane * max_pages + j0 / 16;
+    if constexpr (KV32)
+      attn_f32_item<HD, NT, NW, true>(qrow, (const float *)pool, ptab, min(CH, ctx - j0), layer,
+                                      (size_t)num_layers, kv_dim, h, G, s, qs);
+    else
+      attn_f16_item<HD, NT, NW>(qrow, (const __half *)pool, ptab, min(CH, ctx - j0), layer,
+                                (size_t)num_layers, kv_dim, h, G, s);
     constexpr int RS = 2 + HD;  // floats per record
     const size_t hstride = (size_t)n_chunks_max * RS;
     float *rbase = scratch + ((size_t)m * Hq + qh0) * hstride;
@@ -1702,7 +1680,7 @@ __global__ __launch_bounds__(64 * NW) void attn_o_kernel(AttnOArgs a) {
       if (ch == 0) load_weights();
     };
     if constexpr (KV32)
-      attn_f32_item<HD, NT, NW>(a.q + (size_t)h * SL, (const float *)a.kv_pool, prow + j0 / 16,
+      attn_f32_item<HD, NT, NW, false>(a.q + (size_t)h * SL, (const float *)a.kv_pool, prow + j0 / 16,
                                 min(CH, ctx - j0), a.layer, (size_t)a.num_layers, Hkv * HD, h, G,
                                 s, qs, hook);
     else
@@ -1918,40 +1896,39 @@ __global__ __launch_bounds__(kCombineThreads) void attn_combine2_kernel(
   }
 }
 
-hipError_t launch_attention_f16(const float *q, const void *kv_pool, const int32_t *page_table,
-                                int max_pages, const int32_t *lane_of_row, const int32_t *ctx_len,
-                                int M, int layer, int num_layers, int num_heads, int num_kv_heads,
-                                int head_dim, int max_ctx, float *scratch, float *out,
-                                hipStream_t st, int wp, int nw, PlanesDst emit) {
-  if (num_heads % num_kv_heads != 0 || num_heads / num_kv_heads > kMaxGroup || M < 1 || M > 64 ||
-      max_ctx < 1)
-    return hipErrorInvalidValue;
+// The work-list attention with wp positions per wave and nw waves per item.
+static hipError_t launch_attention_list(const float *q, const void *kv_pool, bool kv_f16,
+                                        const int32_t *page_table, int max_pages,
+                                        const int32_t *lane_of_row, const int32_t *ctx_len, int M,
+                                        int layer, int num_layers, int num_heads,
+                                        int num_kv_heads, int head_dim, int max_ctx,
+                                        float *scratch, float *out, hipStream_t st, int wp, int nw,
+                                        PlanesDst emit) {
   const int chunk = wp * nw;
-  if (chunk < kF16MinChunk || wp % 16) return hipErrorInvalidValue;
   const int nch = (max_ctx + chunk - 1) / chunk;  // record slots per (row, query head)
-  if (nch > kMaxRecords) return hipErrorInvalidValue;
   // one workgroup per work item up to a cap; the rest loop over the list
   const long items = (long)nch * num_kv_heads * M;
   const unsigned grid = (unsigned)std::min<long>(items, kAttnMaxGrid);
-  const __half *pool = (const __half *)kv_pool;
-#define GK_F16(HD, NT, NW)                                                                   \
-  hipLaunchKernelGGL((attn_f16_kernel<HD, NT, NW>), dim3(grid), dim3(64 * NW), 0, st, q, pool, \
-                     page_table, max_pages, lane_of_row, ctx_len, M, layer, num_layers,      \
-                     num_heads, num_kv_heads, nch, max_ctx, scratch, out, emit)
-#define GK_F16_HD(NT, NW)                                        \
-  do {                                                          \
-    if (head_dim == 64) GK_F16(64, NT, NW);                     \
-    else if (head_dim == 128) GK_F16(128, NT, NW);              \
-    else return hipErrorInvalidValue;                           \
+#define GK_LIST(HD, NT, NW, KV32)                                                             \
+  hipLaunchKernelGGL((attn_list_kernel<HD, NT, NW, KV32>), dim3(grid), dim3(64 * NW), 0, st, q, \
+                     kv_pool, page_table, max_pages, lane_of_row, ctx_len, M, layer,           \
+                     num_layers, num_heads, num_kv_heads, nch, max_ctx, scratch, out, emit)
+#define GK_LIST_HD(NT, NW, KV32)                                   \
+  do {                                                             \
+    if (head_dim == 64) GK_LIST(64, NT, NW, KV32);                 \
+    else GK_LIST(128, NT, NW, KV32);                               \
   } while (0)
-  if (wp == 16 && nw == 4) GK_F16_HD(1, 4);
-  else if (wp == 16 && nw == 8) GK_F16_HD(1, 8);
-  else if (wp == 16 && nw == 16) GK_F16_HD(1, 16);
-  else if (wp == 32 && nw == 4) GK_F16_HD(2, 4);
-  else if (wp == 32 && nw == 8) GK_F16_HD(2, 8);
-  else return hipErrorInvalidValue;
-#undef GK_F16_HD
-#undef GK_F16
+  if (kv_f16) {
+    if (wp == 16) GK_LIST_HD(1, 4, false);
+    else if (nw == 4) GK_LIST_HD(2, 4, false);
+    else GK_LIST_HD(2, 8, false);
+  } else {
+    if (nw == 16) GK_LIST_HD(1, 16, true);
+    else if (nw == 8) GK_LIST_HD(1, 8, true);
+    else GK_LIST_HD(1, 4, true);
+  }
+#undef GK_LIST_HD
+#undef GK_LIST
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || nch <= 1) return e;
   if (head_dim == 64)
@@ -2240,47 +2217,34 @@ hipError_t launch_attention(const float *q, const void *kv_pool, int kv_f16,
                             float *scratch, float *out, hipStream_t st, PlanesDst emit) {
   if (num_heads % num_kv_heads != 0 || num_heads / num_kv_heads > kMaxGroup)
     return hipErrorInvalidValue;
-  if (kv_f16) {
-    // contexts up to 256 positions: one work item per (row, KV head) of 8
-    // waves x 2 pages, no combine launch; longer ones: 64-position items of
-    // 4 waves x 1 page for few (row, KV head) pairs (batch-1 decode), else
-    // 128-position items of 4 waves x 2 pages (measured at 1-32 rows,
-    // contexts 16-8192)
-    int wp = 32, nw = 8;
-    if (max_ctx > 256) {
-      wp = M * num_kv_heads < 16 ? 16 : 32;
-      nw = 4;
-    }
-    return launch_attention_f16(q, kv_pool, page_table, max_pages, lane_of_row, ctx_len, M, layer,
-                                num_layers, num_heads, num_kv_heads, head_dim, max_ctx, scratch,
-                                out, st, wp, nw, emit);
+  if (head_dim != 64 && head_dim != 128) return hipErrorInvalidValue;
+  // contexts up to 256 positions: one work item per (row, KV head), 8 waves x 2
+  // pages of fp16 or 16 waves x 1 page of f32 (twice the registers a page),
+  // no combine launch; longer ones: 64-position items of 4 waves x 1 page for
+  // few (row, KV head) pairs (batch-1 decode) and for f32, else 128-position
+  // items of 4 waves x 2 pages (fp16 measured at 1-32 rows, contexts 16-8192)
+  int wp = kv_f16 ? 32 : 16, nw = kv_f16 ? 8 : 16;
+  if (max_ctx > 256) {
+    if (M * num_kv_heads < 16) wp = 16;
+    nw = 4;
   }
+  const bool list = M <= 64 && max_ctx >= 1 && (max_ctx + wp * nw - 1) / (wp * nw) <= kMaxRecords;
+  if (kv_f16 && (!list || M < 1)) return hipErrorInvalidValue;
+  if (list && M >= 1)
+    return launch_attention_list(q, kv_pool, kv_f16 != 0, page_table, max_pages, lane_of_row,
+                                 ctx_len, M, layer, num_layers, num_heads, num_kv_heads, head_dim,
+                                 max_ctx, scratch, out, st, wp, nw, emit);
+  // f32 prompt chunks (more rows than a wave can list) and contexts of more
+  // than 65536 positions
   const int chunk = attention_chunk(max_ctx, num_kv_heads, M);
   if ((max_ctx + chunk - 1) / chunk > kMaxRecords) return hipErrorInvalidValue;
   const int nch = (max_ctx + chunk - 1) / chunk;
-  // few workgroups (batch-1 decode, f32 KV): one query head each; fp16 KV
-  // always groups the query heads of a KV head (MFMA scores)
-  const bool per_head = !kv_f16 && nch * num_kv_heads * M < 64;
-  dim3 grid(nch, per_head ? num_heads : num_kv_heads, M);
-#define GK_ATT(HD, F)                                                                           \
-  do {                                                                                          \
-    if (per_head)                                                                               \
-      hipLaunchKernelGGL((attn_decode_kernel<HD, F, 1>), grid, dim3(256), 0, st, q, kv_pool,    \
-                         page_table, max_pages, lane_of_row, ctx_len, layer, num_layers,        \
-                         num_heads, num_kv_heads, chunk, nch, max_ctx, scratch, out, emit);     \
-    else                                                                                        \
-      hipLaunchKernelGGL((attn_decode_kernel<HD, F, kMaxGroup>), grid, dim3(256), 0, st, q,     \
-                         kv_pool, page_table, max_pages, lane_of_row, ctx_len, layer,           \
-                         num_layers, num_heads, num_kv_heads, chunk, nch, max_ctx, scratch, out, \
-                         emit);                                                                 \
-  } while (0)
-  if (head_dim == 64) {
-    if (kv_f16) GK_ATT(64, 1); else GK_ATT(64, 0);
-  } else if (head_dim == 128) {
-    if (kv_f16) GK_ATT(128, 1); else GK_ATT(128, 0);
-  } else {
-    return hipErrorInvalidValue;
-  }
+  const dim3 grid(nch, num_kv_heads, M);
+#define GK_ATT(HD)                                                                               \
+  hipLaunchKernelGGL((attn_decode_kernel<HD>), grid, dim3(256), 0, st, q, (const float *)kv_pool, \
+                     page_table, max_pages, lane_of_row, ctx_len, layer, num_layers, num_heads,  \
+                     num_kv_heads, chunk, nch, max_ctx, scratch, out, emit)
+  if (head_dim == 64) GK_ATT(64); else GK_ATT(128);
 #undef GK_ATT
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || nch <= 1) return e;

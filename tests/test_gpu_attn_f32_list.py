@@ -1,0 +1,71 @@
+"""f32-page decode attention through glacier_hip_paged_attention at the edges
+of its work list: 16-position pages, 64- and 256-position items, the line at
+max_ctx = 256, one and 64 lanes, group sizes 1 to 8, K / V beyond the fp16
+range, unused page slots holding NaN. Against 64-bit sums; bar 1e-6 of the
+largest output (f32 scores of |q . k| up to ~60: 2^-19 absolute before the
+1 / sqrt(hd) factor)."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+LAYERS, LAYER = 2, 1
+
+
+def _run(gh, gctx, ctxs, max_ctx, Hq, Hkv, hd, seed, kv_scale=1.0):
+    import torch
+
+    g = torch.Generator().manual_seed(seed)
+    pages = [-(-c // 16) for c in ctxs]
+    width = -(-max_ctx // 16)
+    perm = torch.randperm(sum(pages) + 1, generator=g)
+    pool = torch.full((sum(pages) + 1, LAYERS, 2, 16, Hkv * hd), float("nan"))
+    pool[perm[-1]] = 0.0
+    table = torch.full((len(ctxs), width), int(perm[-1]), dtype=torch.int32)
+    q = 1.5 * torch.randn((len(ctxs), Hq, hd), generator=g) / kv_scale
+    want = np.empty((len(ctxs), Hq, hd))
+    at = 0
+    for i, c in enumerate(ctxs):
+        kv = kv_scale * torch.randn((2, c, Hkv * hd), generator=g)
+        for p in range(pages[i]):
+            table[i, p] = perm[at + p]
+            n = min(16, c - 16 * p)
+            pool[perm[at + p], LAYER, :, :n] = kv[:, 16 * p:16 * p + n]
+        at += pages[i]
+        k64 = kv.double().view(2, c, Hkv, hd)
+        for h in range(Hq):
+            kh = h // (Hq // Hkv)
+            w = torch.softmax((k64[0, :, kh] @ q[i, h].double()) / np.sqrt(hd), -1)
+            want[i, h] = (w @ k64[1, :, kh]).numpy()
+    qd, pd, td = q.reshape(len(ctxs), -1).cuda(), pool.cuda(), table.cuda()
+    cl = torch.tensor(ctxs, dtype=torch.int32, device="cuda")
+    out = torch.empty_like(qd)
+    torch.cuda.synchronize()
+    gh.check(gh.lib().glacier_hip_paged_attention(
+        gctx.h, qd.data_ptr(), pd.data_ptr(), gh.F32, td.data_ptr(), width, cl.data_ptr(), len(ctxs),
+        LAYER, LAYERS, Hq, Hkv, hd, max_ctx, out.data_ptr(), None), "paged_attention", gctx.h)
+    gctx.sync()
+    err = np.max(np.abs(out.cpu().numpy().reshape(want.shape) - want)) / np.max(np.abs(want))
+    assert err < 1e-6, err
+
+
+@pytest.mark.parametrize("max_ctx", [256, 257])
+@pytest.mark.parametrize("hd", [64, 128])
+def test_context_edges(gh, gctx, hd, max_ctx):
+    _run(gh, gctx, [1, 15, 16, 17, 63, 64, 65, 127, 128, 129, 255, 256, max_ctx], max_ctx, 14, 2, hd, 3)
+
+
+@pytest.mark.parametrize("ctxs", [[1], [3000], [5] * 64, list(range(1, 65)), [2000] + [7] * 20])
+def test_lane_counts(gh, gctx, ctxs):
+    _run(gh, gctx, ctxs, max(ctxs), 8, 2, 64, len(ctxs))
+
+
+@pytest.mark.parametrize("G", [1, 2, 3, 5, 8])
+@pytest.mark.parametrize("hd", [64, 128])
+def test_group_sizes(gh, gctx, G, hd):
+    _run(gh, gctx, [200, 33, 300], 300, 3 * G, 3, hd, G)
+
+
+@pytest.mark.parametrize("scale", [1e6, 1e-6])
+def test_values_outside_the_fp16_range(gh, gctx, scale):
+    _run(gh, gctx, [40, 300], 300, 8, 2, 128, 5, kv_scale=scale)
