@@ -1306,6 +1306,14 @@ static __device__ __forceinline__ void attn_f16_item(const float *qrow, const __
   attn_item_merge<HD, NW>(o, mx, sum, G, s);
 }
 
+// a + b rounded, and exactly what the rounding left out (Knuth's two-sum).
+template <class T>
+static __device__ __forceinline__ T two_sum(T a, T b, T &rest) {
+  const T r = a + b, t = r - a;
+  rest = (a - (r - t)) + (b - t);
+  return r;
+}
+
 // The same work item over f32 KV pages (the reference's KV storage), with
 // the same lane layout, softmax and merge as attn_f16_item, on
 // v_mfma_f32_16x16x16f16 with every f32 operand split into fp16 hi + lo
@@ -1406,7 +1414,7 @@ static __device__ __forceinline__ void attn_f32_item(const float *qrow, const fl
     // lanes of heads past G take q = 0 (their rows are never read)
     const bool qon = j < G;
     const float *qr = qs + (j < G ? j : 0) * HD + c * QD;
-    f4 sc[NT];
+    f4 sc[NT], tail[NT];  // scores; kExact: what their last sums rounded off
 #pragma unroll
     for (int T = 0; T < NT; ++T) {
       f4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -1430,8 +1438,13 @@ static __device__ __forceinline__ void attn_f32_item(const float *qrow, const fl
           acc = __builtin_amdgcn_mfma_f32_16x16x16f16(kl, qh, acc, 0, 0, 0);
         }
       }
-      if constexpr (kExact)
-        acc = ((part[0] + part[1]) + (part[2] + part[3])) + ((part[4] + part[5]) + (part[6] + part[7]));
+      if constexpr (kExact) {
+        const f4 a = part[0] + part[1], b = part[2] + part[3];
+        const f4 e = part[4] + part[5], f = part[6] + part[7];
+        f4 t0, t1, t2;
+        acc = two_sum(two_sum(a, b, t0), two_sum(e, f, t1), t2);
+        tail[T] = t2 + (t0 + t1);
+      }
 #pragma unroll
       for (int rr = 0; rr < 4; ++rr) {
         sc[T][rr] = 16 * T + 4 * c + rr < wn ? (kExact ? acc[rr] : acc[rr] * scale) : -INFINITY;
@@ -1444,8 +1457,21 @@ static __device__ __forceinline__ void attn_f32_item(const float *qrow, const fl
     for (int T = 0; T < NT; ++T)
 #pragma unroll
       for (int rr = 0; rr < 4; ++rr) {
-        // (kExact: the score is not rounded before the maximum is taken off)
-        const float p = expf(kExact ? fmaf(sc[T][rr], scale, -mx) : sc[T][rr] - mx);
+        float p;
+        if constexpr (kExact) {
+          // the exponent as r + err: err is the rounding of r = score - maximum
+          // and the score's tail (at scores of 3, one rounding of q . k alone is
+          // 1e-7 of p; the kernel waits for memory, not for these). r of -inf
+          // (masked) keeps its 0.
+          const float r = fmaf(sc[T][rr], scale, -mx);
+          float de;
+          const float d = two_sum(mx, r, de);
+          const float err = (fmaf(sc[T][rr], scale, -d) - de) + tail[T][rr] * scale;
+          p = expf(r);
+          if (r > -128.0f) p = fmaf(p, err, p);
+        } else {
+          p = expf(sc[T][rr] - mx);
+        }
         sc[T][rr] = p;
         sum += p;
       }
@@ -1518,7 +1544,9 @@ static __device__ __forceinline__ void attn_f32_item(const float *qrow, const fl
 // f32 pages run the same list with attn_f32_item, one page per wave and f32
 // MFMAs; bound by the latency of the page walk and the loads behind it. 6 lanes
 // of 14 / 2 heads of 64 at contexts 37 to 4096: 18.4 us with attn_decode_kernel
-// (scalar dots, 512-position chunks) -> 8.9.
+// (scalar dots, 512-position chunks) -> 9.3; the compensated exponents cost 0.2 of
+// them and take the mean error against 64 bits from 1.77e-7 to 1.42e-7 (1.67e-7 with
+// attn_decode_kernel).
 // ---------------------------------------------------------------------------
 template <int HD, int NT, int NW, bool KV32>
 __global__ __launch_bounds__(64 * NW) void attn_list_kernel(
@@ -1579,7 +1607,7 @@ __global__ __launch_bounds__(64 * NW) void attn_list_kernel(
         O = fmaf(s.so[w][g][d], f, O);
       }
       if (nch == 1) {
-        const float v = O * (1.0f / L);
+        const float v = KV32 ? O / L : O * (1.0f / L);
         out[((size_t)m * Hq + qh0 + g) * HD + d] = v;
         emit_group(pd, v, t & 31, ((qh0 + g) * HD + d) >> 5, m, M);
       } else {
@@ -1924,7 +1952,6 @@ static hipError_t launch_attention_list(const float *q, const void *kv_pool, boo
     else GK_LIST_HD(2, 8, false);
   } else {
     if (nw == 16) GK_LIST_HD(1, 16, true);
-    else if (nw == 8) GK_LIST_HD(1, 8, true);
     else GK_LIST_HD(1, 4, true);
   }
 #undef GK_LIST_HD
