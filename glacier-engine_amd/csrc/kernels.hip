@@ -1414,7 +1414,7 @@ static __device__ __forceinline__ void attn_f32_item(const float *qrow, const fl
     // lanes of heads past G take q = 0 (their rows are never read)
     const bool qon = j < G;
     const float *qr = qs + (j < G ? j : 0) * HD + c * QD;
-    f4 sc[NT], tail[NT];  // scores; kExact: what their last sums rounded off
+    f4 sc[NT], tail[NT];  // scores; kExact: what their last roundings left out
 #pragma unroll
     for (int T = 0; T < NT; ++T) {
       f4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -1447,28 +1447,30 @@ static __device__ __forceinline__ void attn_f32_item(const float *qrow, const fl
       }
 #pragma unroll
       for (int rr = 0; rr < 4; ++rr) {
-        sc[T][rr] = 16 * T + 4 * c + rr < wn ? (kExact ? acc[rr] : acc[rr] * scale) : -INFINITY;
+        const float v = acc[rr] * scale;
+        if constexpr (kExact) tail[T][rr] = fmaf(tail[T][rr], scale, fmaf(acc[rr], scale, -v));
+        sc[T][rr] = 16 * T + 4 * c + rr < wn ? v : -INFINITY;
         mx = fmaxf(mx, sc[T][rr]);
       }
     }
     mx = xor32_max(xor16_max(mx));
-    if constexpr (kExact) mx *= scale;
 #pragma unroll
     for (int T = 0; T < NT; ++T)
 #pragma unroll
       for (int rr = 0; rr < 4; ++rr) {
         float p;
         if constexpr (kExact) {
-          // the exponent as r + err: err is the rounding of r = score - maximum
-          // and the score's tail (at scores of 3, one rounding of q . k alone is
-          // 1e-7 of p; the kernel waits for memory, not for these). r of -inf
-          // (masked) keeps its 0.
-          const float r = fmaf(sc[T][rr], scale, -mx);
+          // the exponent as r + err: err is what the subtraction and the score
+          // rounded off (at scores of 3, one rounding of q . k alone is 1e-7
+          // of p; the kernel waits for memory, not for these). 1 + err stands
+          // for exp(err) while err is small; where scores are so large that it
+          // is not (or infinite: err is NaN, and a masked -inf keeps its 0)
+          // the weight is the rounded score's, never negative.
           float de;
-          const float d = two_sum(mx, r, de);
-          const float err = (fmaf(sc[T][rr], scale, -d) - de) + tail[T][rr] * scale;
+          const float r = two_sum(sc[T][rr], -mx, de);
+          const float err = de + tail[T][rr];
           p = expf(r);
-          if (r > -128.0f) p = fmaf(p, err, p);
+          if (fabsf(err) < 0x1p-8f) p = fmaf(p, err, p);
         } else {
           p = expf(sc[T][rr] - mx);
         }

@@ -69,3 +69,45 @@ def test_group_sizes(gh, gctx, G, hd):
 @pytest.mark.parametrize("scale", [1e6, 1e-6])
 def test_values_outside_the_fp16_range(gh, gctx, scale):
     _run(gh, gctx, [40, 300], 300, 8, 2, 128, 5, kv_scale=scale)
+
+
+def _uniform(gh, gctx, q, k, v, hd):
+    """One lane, one KV head, two query heads: q [2][hd], k and v [c][hd]."""
+    import torch
+
+    c = k.shape[0]
+    pages = -(-c // 16)
+    pool = torch.zeros((pages, 1, 2, 16, hd))
+    for p in range(c):
+        pool[p // 16, 0, 0, p % 16] = k[p]
+        pool[p // 16, 0, 1, p % 16] = v[p]
+    qd, pd = q.reshape(1, -1).cuda(), pool.cuda()
+    td = torch.arange(pages, dtype=torch.int32, device="cuda").view(1, -1)
+    cl = torch.tensor([c], dtype=torch.int32, device="cuda")
+    out = torch.empty_like(qd)
+    torch.cuda.synchronize()
+    gh.check(gh.lib().glacier_hip_paged_attention(
+        gctx.h, qd.data_ptr(), pd.data_ptr(), gh.F32, td.data_ptr(), pages, cl.data_ptr(), 1, 0, 1, 2,
+        1, hd, c, out.data_ptr(), None), "paged_attention", gctx.h)
+    gctx.sync()
+    return out.cpu().view(2, hd)
+
+
+@pytest.mark.parametrize("size", [1.0, 3e4, 1e15])
+@pytest.mark.parametrize("c", [33, 300])
+@pytest.mark.parametrize("hd", [64, 128])
+def test_equal_scores_of_any_size_weigh_equally(gh, gctx, hd, c, size):
+    """Equal K rows: the output is V's mean whatever their score is, also
+    where one f32 rounding of q . k is worth many e-folds (bar: f32 sums of c
+    equal weights)."""
+    import torch
+
+    for seed in range(6):
+        g = torch.Generator().manual_seed(seed)
+        q = size * torch.randn((2, hd), generator=g)
+        k = size * torch.randn((1, hd), generator=g).repeat(c, 1)
+        v = 1.0 + torch.rand((c, hd), generator=g)
+        want = v.double().mean(0)
+        got = _uniform(gh, gctx, q, k, v, hd).double()
+        err = float((got - want).abs().max())
+        assert err < 2e-6, (seed, err)
