@@ -1454,6 +1454,9 @@ static __device__ __forceinline__ void attn_f32_item(const float *qrow, const fl
       }
     }
     mx = xor32_max(xor16_max(mx));
+    // (scores that all overflowed to -inf: the wave weighs nothing, and its
+    // -inf - -inf must not reach the other waves' sums as NaN)
+    const float m0 = kExact && mx == -INFINITY ? 0.0f : mx;
 #pragma unroll
     for (int T = 0; T < NT; ++T)
 #pragma unroll
@@ -1467,12 +1470,12 @@ static __device__ __forceinline__ void attn_f32_item(const float *qrow, const fl
           // is not (or infinite: err is NaN, and a masked -inf keeps its 0)
           // the weight is the rounded score's, never negative.
           float de;
-          const float r = two_sum(sc[T][rr], -mx, de);
+          const float r = two_sum(sc[T][rr], -m0, de);
           const float err = de + tail[T][rr];
           p = expf(r);
           if (fabsf(err) < 0x1p-8f) p = fmaf(p, err, p);
         } else {
-          p = expf(sc[T][rr] - mx);
+          p = expf(sc[T][rr] - m0);
         }
         sc[T][rr] = p;
         sum += p;

@@ -111,3 +111,27 @@ def test_equal_scores_of_any_size_weigh_equally(gh, gctx, hd, c, size):
         got = _uniform(gh, gctx, q, k, v, hd).double()
         err = float((got - want).abs().max())
         assert err < 2e-6, (seed, err)
+
+
+@pytest.mark.parametrize("c", [64, 300])
+@pytest.mark.parametrize("hd", [64, 128])
+def test_pages_of_minus_infinite_scores_weigh_nothing(gh, gctx, hd, c):
+    """Whole pages whose scores overflow to -inf beside finite ones."""
+    import torch
+
+    g = torch.Generator().manual_seed(c)
+    q = torch.randn((2, hd), generator=g).abs() + 1.0
+    k = torch.randn((c, hd), generator=g)
+    v = torch.randn((c, hd), generator=g)
+    dead = torch.zeros(c, dtype=torch.bool)
+    dead[16:48] = True
+    if c > 128:
+        dead[64:128] = True  # a whole work item
+    k[dead] = -3e38
+    got = _uniform(gh, gctx, q, k, v, hd).double()
+    live = ~dead
+    for h in range(2):
+        sc = (k[live].double() @ q[h].double()) / np.sqrt(hd)
+        want = torch.softmax(sc, -1) @ v[live].double()
+        err = float((got[h] - want).abs().max() / want.abs().max())
+        assert err < 1e-6, (h, err)
