@@ -2015,8 +2015,11 @@ hipError_t launch_attn_o(const AttnOArgs &a, hipStream_t st) {
 // of v), fp16 KV pages.
 //
 // Workgroup = the G query heads of one KV head x R tiles of 16 query rows, a
-// wave each (R = 8 / G, so small groups still share every K/V read among
-// about 8 waves). It walks the keys 32 (two pages) at a time, staged in LDS
+// wave each: as few tiles as fill 4 waves while the grid is at most one
+// workgroup a CU, else R = 8 / G, so small groups still share every K/V read
+// among about 8 waves (32 / 8 heads of 128, fewest tiles against 8 / G: 64
+// rows 7.5 and 9.7 us, 200 after 700 positions 38 and 41; 8 / 8 heads at 2048
+// rows 76 and 84). It walks the keys 32 (two pages) at a time, staged in LDS
 // double buffered with one barrier per 32 keys: K rows, and V transposed (4
 // keys x 4 dims per thread through byte permutes and 8-byte writes). Per 32
 // keys and wave:
@@ -2036,16 +2039,24 @@ hipError_t launch_attn_o(const AttnOArgs &a, hipStream_t st) {
 // rows of 28 / 4 heads of 128: 97 us. 285 us before, with 16 keys a barrier,
 // K = 16 MFMAs, O rescaled and row factors exchanged every 16 keys and V
 // transposed through 2-byte writes.
+// Short prompts (one to three stages) are bound by the chain from the launch
+// to the stores: no integer division in front of the first loads, and one
+// division a row at the end (17 to 100 rows: 0.2 to 0.5 us each).
 // Order: workgroup b takes the b-th longest block, every second run of 256
 // reversed, so a CU's two workgroups are a long and a short one.
 // ---------------------------------------------------------------------------
 constexpr int kPfKeys = 32;
-template <int HD, int KPP>
-__global__ __launch_bounds__(64 * kMaxGroup, 4) void attn_prefill_kernel(
+constexpr int kPfSpread = 256;  // workgroups of fewest tiles, at most one a CU
+// kTileWaves: 0 for one tile, else the most waves (4 waves may take more
+// registers: no second workgroup has to fit beside two others)
+template <int HD, int KPP, int kTileWaves>
+__global__ __launch_bounds__(64 * (kTileWaves ? kTileWaves : kMaxGroup),
+                             kTileWaves == 4 ? 3 : 4) void attn_prefill_kernel(
     const float *q, const __half *pool, const int32_t *ptab, int pos0, int T, int layer,
-    int num_layers, int Hq, int Hkv, int R, float *out) {
+    int num_layers, int Hq, int Hkv, int G, int R, int nqb, float *out) {
   typedef _Float16 h8 __attribute__((ext_vector_type(8)));
   typedef float f4 __attribute__((ext_vector_type(4)));
+  constexpr bool kTiles = kTileWaves > 0;
   constexpr int S = HD / 32;            // steps over the head dim (scores)
   constexpr int NT = HD / 16;           // 16-wide output tiles over the head dim
   constexpr int KP = HD + 8;            // K row stride in halves (padded)
@@ -2057,15 +2068,23 @@ __global__ __launch_bounds__(64 * kMaxGroup, 4) void attn_prefill_kernel(
   const int t = threadIdx.x, l = t & 63, nthr = (int)blockDim.x;
   const int wv = __builtin_amdgcn_readfirstlane(t >> 6);
   const int c = l >> 4, j = l & 15;
-  const int G = Hq / Hkv;
-  const int BQ = 16 * R, nqb = (T + BQ - 1) / BQ;
-  // longest blocks first, every second run of 256 reversed
-  const int W = (int)gridDim.x, b = (int)blockIdx.x, run = b >> 8;
-  const int rank = run & 1 ? 256 * run + min(256, W - 256 * run) - 1 - (b & 255) : b;
-  const int h = rank % Hkv;
-  const int i0 = (nqb - 1 - rank / Hkv) * BQ + 16 * (wv / G);  // this wave's rows
-  const int last_row = min((nqb - rank / Hkv) * BQ, T) - 1;    // the workgroup's
-  const int qh = h * G + wv % G;
+  const int BQ = kTiles ? 16 * R : 16;
+  // longest blocks first, every second run of 256 reversed (the grid's order
+  // itself is the first run: no division in front of a short prompt's loads)
+  const int b = (int)blockIdx.y * Hkv + (int)blockIdx.x, run = b >> 8;
+  int blk = (int)blockIdx.y, h = (int)blockIdx.x;
+  if (run & 1) {
+    const int rank = 256 * run + min(256, Hkv * nqb - 256 * run) - 1 - (b & 255);
+    blk = rank / Hkv;
+    h = rank - blk * Hkv;
+  }
+  int tile = 0, head = wv;  // of this wave
+  if (kTiles)
+    for (; head >= G; head -= G) ++tile;
+  const int i0_wg = (nqb - 1 - blk) * BQ;         // the workgroup's rows
+  const int i0 = i0_wg + 16 * tile;               // this wave's
+  const int last_row = min(i0_wg + BQ, T) - 1;    // the workgroup's
+  const int qh = h * G + head;
   const int kv_dim = Hkv * HD;
   const size_t lay = (size_t)num_layers;
   const int last_pos = pos0 + last_row;
@@ -2210,12 +2229,19 @@ __global__ __launch_bounds__(64 * kMaxGroup, 4) void attn_prefill_kernel(
   }
   // lane (c, j): O[row j][dims 16 nt + 4 c .. + 3]
   sum = xor32_add(xor16_add(sum));
+  // x / sum as the rounded reciprocal and one correction (the quotient's
+  // rounding; the fixup keeps infinities)
+  const float rs = 1.0f / sum;
+  const auto over = [&](float x) {
+    const float y = x * rs;
+    return __builtin_amdgcn_div_fixupf(fmaf(fmaf(-y, sum, x), rs, y), sum, x);
+  };
   if (i0 + j < T) {
     float *orow = out + ((size_t)(i0 + j) * Hq + qh) * HD;
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt)
       *(f4 *)(orow + 16 * nt + 4 * c) =
-          f4{o[nt][0] / sum, o[nt][1] / sum, o[nt][2] / sum, o[nt][3] / sum};
+          f4{over(o[nt][0]), over(o[nt][1]), over(o[nt][2]), over(o[nt][3])};
   }
 }
 
@@ -2228,16 +2254,37 @@ hipError_t launch_attention_prefill(const float *q, const void *kv_pool, const i
     return hipErrorInvalidValue;
   const int G = num_heads / num_kv_heads;
   if (head_dim != 64 && head_dim != 128) return hipErrorInvalidValue;
-  const int R = kMaxGroup / G;  // 320 to 512 threads
-  const dim3 grid((T + 16 * R - 1) / (16 * R) * num_kv_heads), block(64 * G * R);
+  constexpr int kRows = 1 << 19;  // of a launch (its blocks are grid.y, 65535 at most)
+  if (T > kRows) {
+    const hipError_t e =
+        launch_attention_prefill(q, kv_pool, page_table, max_pages, lane, pos0, kRows, layer,
+                                 num_layers, num_heads, num_kv_heads, head_dim, out, st);
+    const size_t done = (size_t)kRows * num_heads * head_dim;
+    return e != hipSuccess ? e
+                           : launch_attention_prefill(q + done, kv_pool, page_table, max_pages,
+                                                      lane, pos0 + kRows, T - kRows, layer,
+                                                      num_layers, num_heads, num_kv_heads, head_dim,
+                                                      out + done, st);
+  }
+  int R = (4 + G - 1) / G;  // 256 threads or more (the V staging's blocks)
+  if ((long)(T + 16 * R - 1) / (16 * R) * num_kv_heads > kPfSpread) R = kMaxGroup / G;
+  const int nqb = (T + 16 * R - 1) / (16 * R);
+  const dim3 grid(num_kv_heads, nqb), block(64 * G * R);
   const int32_t *ptab = page_table + (size_t)lane * max_pages;
   const __half *pool = (const __half *)kv_pool;
-#define GK_PF(HD, P)                                                                             \
-  hipLaunchKernelGGL((attn_prefill_kernel<HD, P>), grid, block, 0, st, q, pool, ptab, pos0, T,   \
-                     layer, num_layers, num_heads, num_kv_heads, R, out)
-  if (head_dim == 64) GK_PF(64, 1);
-  else if (block.x == 64 * kMaxGroup) GK_PF(128, 1);
-  else GK_PF(128, 2);
+#define GK_PF(HD, P, TW)                                                                          \
+  hipLaunchKernelGGL((attn_prefill_kernel<HD, P, TW>), grid, block, 0, st, q, pool, ptab, pos0, T, \
+                     layer, num_layers, num_heads, num_kv_heads, G, R, nqb, out)
+  const int waves = G * R;
+  if (head_dim == 64) {
+    if (R > 1) GK_PF(64, 1, 8); else GK_PF(64, 1, 0);
+  } else if (waves == 8) {
+    if (R > 1) GK_PF(128, 1, 8); else GK_PF(128, 1, 0);
+  } else if (R == 1) {
+    GK_PF(128, 2, 0);
+  } else {
+    if (waves == 4) GK_PF(128, 2, 4); else GK_PF(128, 2, 6);
+  }
 #undef GK_PF
   return hipGetLastError();
 }

@@ -66,3 +66,11 @@ def test_group_sizes(gh, gctx, G, hd):
 def test_more_workgroups_than_a_run(gh, gctx):
     """Over 512 workgroups (three runs of 256 in the block order)."""
     _case(gh, gctx, 40, 8, 64, 5, 1100, 7)
+
+
+@pytest.mark.parametrize("G,T", [(1, 400), (1, 530), (2, 250), (2, 290), (3, 150), (4, 100), (4, 150)])
+@pytest.mark.parametrize("hd", [64, 128])
+def test_tiles_per_workgroup(gh, gctx, G, T, hd):
+    """32 KV heads: row counts on both sides of the line (256 workgroups of
+    fewest tiles) past which a workgroup takes 8 / G tiles."""
+    _case(gh, gctx, 32 * G, 32, hd, 21, T, G)
