@@ -2089,6 +2089,9 @@ __global__ __launch_bounds__(64 * (kTileWaves ? kTileWaves : kMaxGroup),
   const size_t lay = (size_t)num_layers;
   const int last_pos = pos0 + last_row;
   const int nst = last_pos / kPfKeys + 1;
+  const int wave_last = pos0 + min(i0 + 15, T - 1);  // of this wave's rows
+  // kTiles: the first stage with keys past the workgroup's first tile
+  const int edge_st = (pos0 + i0_wg + 16) / kPfKeys;
   const float cl2 = 1.44269504088896341f / sqrtf((float)HD);
 
   // staging: this thread's K pieces t + nthr i and V block t; keys past the
@@ -2140,6 +2143,18 @@ __global__ __launch_bounds__(64 * (kTileWaves ? kTileWaves : kMaxGroup),
       }
     }
   };
+  // kTiles: whether V, past some tile, is not all finite
+  __shared__ int unfinite;
+  if (kTiles && t == 0) unfinite = 0;
+  const auto note = [&]() {
+    uint32_t top = 0;  // the largest exponent of this thread's halves
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+#pragma unroll
+      for (int e = 0; e < 2; ++e)
+        top = max(max(top, vreg[k][e] & 0x7C00u), (vreg[k][e] >> 16) & 0x7C00u);
+    if (t < VBLOCKS && top == 0x7C00u) unfinite = 1;
+  };
   fetch(0);
 
   // Q^T as the B operand: lane (c, j) = row i0 + j, dims 32 st + 8 c .. + 7
@@ -2162,70 +2177,99 @@ __global__ __launch_bounds__(64 * (kTileWaves ? kTileWaves : kMaxGroup),
   stage(0);
   const int qpos = pos0 + i0 + j;  // position of this lane's row
   f4 o[NT];
+  float mx, sum;
+  // The walk over the staged keys. A weight of 0 times an infinity is not 0:
+  // where V past one of a workgroup's tiles is not all finite, a second,
+  // masked walk zeroes the V rows past each wave's last (a walk that always
+  // masks: 10% slower at 2048 rows of 32 / 8 heads of 128).
+  const auto walk = [&](auto masked) {
 #pragma unroll
-  for (int nt = 0; nt < NT; ++nt) o[nt] = f4{0.0f, 0.0f, 0.0f, 0.0f};
-  float mx = -INFINITY, sum = 0.0f;
-  __syncthreads();
-
-  for (int st = 0; st < nst; ++st) {
-    const int bi = st & 1;
-    if (st + 1 < nst) fetch(st + 1);  // the next keys in flight
-    f4 acc[2];
-#pragma unroll
-    for (int tt = 0; tt < 2; ++tt) {
-      acc[tt] = f4{0.0f, 0.0f, 0.0f, 0.0f};
-      h8 kf[S];
-#pragma unroll
-      for (int s2 = 0; s2 < S; ++s2)
-        kf[s2] = *(const h8 *)&ks[bi][(16 * tt + j) * KP + 32 * s2 + 8 * c];
-#pragma unroll
-      for (int s2 = 0; s2 < S; ++s2)  // (the small terms first: fewer roundings at full size)
-        acc[tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[s2], qlo[s2], acc[tt], 0, 0, 0);
-#pragma unroll
-      for (int s2 = 0; s2 < S; ++s2)
-        acc[tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[s2], qhi[s2], acc[tt], 0, 0, 0);
-    }
-    float sv[8], pm = -INFINITY;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) sv[e] = acc[e >> 2][e & 3];
-    if (st * kPfKeys + kPfKeys - 1 > pos0 + i0) {  // the causal edge passes here (uniform)
-#pragma unroll
-      for (int e = 0; e < 8; ++e)
-        if (st * kPfKeys + 16 * (e >> 2) + 4 * c + (e & 3) > qpos) sv[e] = -INFINITY;
-    }
-#pragma unroll
-    for (int e = 0; e < 8; ++e) pm = fmaxf(pm, sv[e]);
-    pm = xor32_max(xor16_max(pm));
-    // (a row past the workgroup's keys keeps its finite maximum: key 0 is in
-    // every row's range)
-    if (__any(pm > mx)) {
-      const float mnew = fmaxf(mx, pm);
-      const float alpha = __builtin_amdgcn_exp2f((mx - mnew) * cl2);
-      sum *= alpha;
-#pragma unroll
-      for (int nt = 0; nt < NT; ++nt) o[nt] *= alpha;
-      mx = mnew;
-    }
-    const float m2 = mx * cl2;
-    h8 phi, plo;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const float pv = __builtin_amdgcn_exp2f(fmaf(sv[e], cl2, -m2));
-      sum += pv;
-      const _Float16 hv = (_Float16)pv;
-      phi[e] = hv;
-      plo[e] = (_Float16)(pv - (float)hv);
-    }
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt) {
-      const h8 vf = *(const h8 *)&vt[bi][(16 * nt + j) * VP + 8 * c];
-      o[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf, phi, o[nt], 0, 0, 0);
-      o[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf, plo, o[nt], 0, 0, 0);
-    }
-    // publish the next keys (the other buffer was last read before the
-    // previous barrier)
-    if (st + 1 < nst) stage(bi ^ 1);
+    for (int nt = 0; nt < NT; ++nt) o[nt] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+    mx = -INFINITY;
+    sum = 0.0f;
     __syncthreads();
+    for (int st = 0; st < nst; ++st) {
+      const int bi = st & 1;
+      if (kTiles && !masked && st >= edge_st) note();
+      if (!masked && st + 1 < nst) fetch(st + 1);  // the next keys in flight
+      f4 acc[2];
+#pragma unroll
+      for (int tt = 0; tt < 2; ++tt) {
+        acc[tt] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+        h8 kf[S];
+#pragma unroll
+        for (int s2 = 0; s2 < S; ++s2)
+          kf[s2] = *(const h8 *)&ks[bi][(16 * tt + j) * KP + 32 * s2 + 8 * c];
+#pragma unroll
+        for (int s2 = 0; s2 < S; ++s2)  // (the small terms first: fewer roundings at full size)
+          acc[tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[s2], qlo[s2], acc[tt], 0, 0, 0);
+#pragma unroll
+        for (int s2 = 0; s2 < S; ++s2)
+          acc[tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[s2], qhi[s2], acc[tt], 0, 0, 0);
+      }
+      float sv[8], pm = -INFINITY;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) sv[e] = acc[e >> 2][e & 3];
+      if (st * kPfKeys + kPfKeys - 1 > pos0 + i0) {  // the causal edge passes here (uniform)
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          if (st * kPfKeys + 16 * (e >> 2) + 4 * c + (e & 3) > qpos) sv[e] = -INFINITY;
+      }
+#pragma unroll
+      for (int e = 0; e < 8; ++e) pm = fmaxf(pm, sv[e]);
+      pm = xor32_max(xor16_max(pm));
+      // (a row past the workgroup's keys keeps its finite maximum: key 0 is in
+      // every row's range)
+      if (__any(pm > mx)) {
+        const float mnew = fmaxf(mx, pm);
+        const float alpha = __builtin_amdgcn_exp2f((mx - mnew) * cl2);
+        sum *= alpha;
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) o[nt] *= alpha;
+        mx = mnew;
+      }
+      const float m2 = mx * cl2;
+      h8 phi, plo;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float pv = __builtin_amdgcn_exp2f(fmaf(sv[e], cl2, -m2));
+        sum += pv;
+        const _Float16 hv = (_Float16)pv;
+        phi[e] = hv;
+        plo[e] = (_Float16)(pv - (float)hv);
+      }
+      v4u keep;  // of this lane's keys 16 T + 4 c + r, as pairs of halves
+#pragma unroll
+      for (int d = 0; d < 4; ++d) {
+        const int past = st * kPfKeys + 16 * (d >> 1) + 4 * c + 2 * (d & 1) - wave_last;
+        keep[d] = past > 0 ? 0u : past == 0 ? 0xFFFFu : ~0u;
+      }
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt) {
+        v4u vraw = *(const v4u *)&vt[bi][(16 * nt + j) * VP + 8 * c];
+        if constexpr (masked) vraw &= keep;
+        const h8 vf = __builtin_bit_cast(h8, vraw);
+        o[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf, phi, o[nt], 0, 0, 0);
+        o[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf, plo, o[nt], 0, 0, 0);
+      }
+      // publish the next keys (the other buffer was last read before the
+      // previous barrier)
+      if (st + 1 < nst) {
+        if (masked) fetch(st + 1);  // (rare: its loads need not hold registers above)
+        stage(bi ^ 1);
+      }
+      __syncthreads();
+    }
+  };
+  walk(std::false_type());
+  if constexpr (kTiles) {
+    if (unfinite) {
+      pg0 = page(0);
+      pg1 = page(1);
+      fetch(0);
+      stage(0);
+      walk(std::true_type());
+    }
   }
   // lane (c, j): O[row j][dims 16 nt + 4 c .. + 3]
   sum = xor32_add(xor16_add(sum));

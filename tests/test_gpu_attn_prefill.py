@@ -74,3 +74,46 @@ def test_tiles_per_workgroup(gh, gctx, G, T, hd):
     """32 KV heads: row counts on both sides of the line (256 workgroups of
     fewest tiles) past which a workgroup takes 8 / G tiles."""
     _case(gh, gctx, 32 * G, 32, hd, 21, T, G)
+
+
+def _launch(gh, gctx, q, kv, pos0, Hq, Hkv, hd):
+    """q [T][Hq][hd] f32, kv [2][pos0 + T][Hkv * hd] fp16 in consecutive pages."""
+    import torch
+
+    T, end = q.shape[0], kv.shape[1]
+    npages = -(-end // 16)
+    pool = torch.zeros((npages, LAYERS, 2, 16, Hkv * hd), dtype=torch.float16)
+    for p in range(end):
+        pool[p // 16, LAYER, :, p % 16] = kv[:, p]
+    qd, pd = q.reshape(T, -1).cuda(), pool.cuda()
+    td = torch.arange(npages, dtype=torch.int32, device="cuda")
+    out = torch.empty_like(qd)
+    torch.cuda.synchronize()
+    gh.check(gh.lib().glacier_hip_paged_attention_prefill(
+        gctx.h, qd.data_ptr(), pd.data_ptr(), td.data_ptr(), npages, pos0, T, LAYER, LAYERS, Hq, Hkv,
+        hd, out.data_ptr(), None), "attention_prefill", gctx.h)
+    gctx.sync()
+    return out.cpu().view(T, Hq, hd)
+
+
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("G", [1, 2, 3, 4, 7])
+@pytest.mark.parametrize("pos0", [0, 5])
+@pytest.mark.parametrize("bad", [20, 50, 77])
+def test_infinite_v_stays_out_of_earlier_rows(gh, gctx, hd, G, pos0, bad):
+    """An infinity in one position's V row reaches no 16-row tile that ends
+    before that position, wherever both lie in a workgroup's rows and a
+    32-key stage."""
+    import torch
+
+    T, Hkv = 130, 2
+    Hq = G * Hkv
+    g = torch.Generator().manual_seed(G + bad)
+    kv = torch.randn((2, pos0 + T, Hkv * hd), generator=g).half()
+    q = 1.5 * torch.randn((T, Hq, hd), generator=g)
+    want = _launch(gh, gctx, q, kv, pos0, Hq, Hkv, hd)
+    kv[1, pos0 + bad] = float("inf")
+    got = _launch(gh, gctx, q, kv, pos0, Hq, Hkv, hd)
+    before = bad // 16 * 16
+    assert torch.equal(got[:before], want[:before])
+    assert not torch.isfinite(got[bad:]).any()
