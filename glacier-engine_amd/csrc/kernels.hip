@@ -2177,7 +2177,7 @@ __global__ __launch_bounds__(64 * (kTileWaves ? kTileWaves : kMaxGroup),
   stage(0);
   const int qpos = pos0 + i0 + j;  // position of this lane's row
   f4 o[NT];
-  float mx, sum;
+  float m2, sum;
   // The walk over the staged keys. A weight of 0 times an infinity is not 0:
   // where V past one of a workgroup's tiles is not all finite, a second,
   // masked walk zeroes the V rows past each wave's last (a walk that always
@@ -2185,7 +2185,7 @@ __global__ __launch_bounds__(64 * (kTileWaves ? kTileWaves : kMaxGroup),
   const auto walk = [&](auto masked) {
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) o[nt] = f4{0.0f, 0.0f, 0.0f, 0.0f};
-    mx = -INFINITY;
+    m2 = -INFINITY;
     sum = 0.0f;
     __syncthreads();
     for (int st = 0; st < nst; ++st) {
@@ -2219,16 +2219,17 @@ __global__ __launch_bounds__(64 * (kTileWaves ? kTileWaves : kMaxGroup),
       for (int e = 0; e < 8; ++e) pm = fmaxf(pm, sv[e]);
       pm = xor32_max(xor16_max(pm));
       // (a row past the workgroup's keys keeps its finite maximum: key 0 is in
-      // every row's range)
-      if (__any(pm > mx)) {
-        const float mnew = fmaxf(mx, pm);
-        const float alpha = __builtin_amdgcn_exp2f((mx - mnew) * cl2);
+      // every row's range. The state is the rounded product m c that the
+      // weights are taken from, so its rounding cancels in O / sum)
+      const float p2 = pm * cl2;
+      if (__any(p2 > m2)) {
+        const float mnew = fmaxf(m2, p2);
+        const float alpha = __builtin_amdgcn_exp2f(m2 - mnew);
         sum *= alpha;
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) o[nt] *= alpha;
-        mx = mnew;
+        m2 = mnew;
       }
-      const float m2 = mx * cl2;
       h8 phi, plo;
 #pragma unroll
       for (int e = 0; e < 8; ++e) {

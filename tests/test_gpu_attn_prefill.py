@@ -117,3 +117,36 @@ def test_infinite_v_stays_out_of_earlier_rows(gh, gctx, hd, G, pos0, bad):
     before = bad // 16 * 16
     assert torch.equal(got[:before], want[:before])
     assert not torch.isfinite(got[bad:]).any()
+
+
+@pytest.mark.parametrize("top", [50, 200])
+@pytest.mark.parametrize("hd", [64, 128])
+def test_growing_maxima_at_large_scores(gh, gctx, hd, top):
+    """Scores that rise to `top` over the keys, so every 32-key stage raises
+    the maximum of rows whose earlier keys still weigh. Only one dimension is
+    nonzero and its products have 22 bits, so every q . k is exact and the
+    error left is the softmax's own. Bar 1e-6: weights carry the fp16 hi + lo
+    split (2^-22), the exponential (2^-23) and their exponent's rounding, which
+    averages under 2^-22 over the keys that count (the nearest few e-folds); a
+    rescale that does not match the rounded maxima the weights were taken from
+    costs about half an ulp of 1.44 * top (3e-6 to 5e-6 here at 200)."""
+    import torch
+
+    T, Hq, Hkv = 300, 4, 2
+    g = torch.Generator().manual_seed(top + hd)
+    unit = top * hd ** 0.5 / 32.0  # K at which a q of 32 scores `top`
+    q = torch.zeros((T, Hq, hd))
+    q[:, :, 0] = (30 + 4 * torch.rand((T, Hq), generator=g)).half().float()
+    kv = torch.randn((2, T, Hkv, hd), generator=g).half()
+    kv[0] = 0
+    rise = unit * (1 - 0.08 * (50 / top) * (T - torch.arange(T)) / 32)
+    kv[0, :, :, 0] = (rise[:, None] + 0.02 * unit * (50 / top) *
+                      torch.randn((T, Hkv), generator=g)).half()
+    got = _launch(gh, gctx, q, kv.reshape(2, T, -1), 0, Hq, Hkv, hd).double()
+    mask = torch.arange(T)[None, :] > torch.arange(T)[:, None]
+    for h in range(Hq):
+        K, V = kv[0, :, h // 2].double(), kv[1, :, h // 2].double()
+        sc = (q[:, h].double() @ K.T) / np.sqrt(hd)
+        want = torch.softmax(sc.masked_fill(mask, -np.inf), -1) @ V
+        err = float((got[:, h] - want).abs().max() / want.abs().max())
+        assert err < 1e-6, (h, err)
