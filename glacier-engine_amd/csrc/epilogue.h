@@ -59,6 +59,15 @@ static __device__ __forceinline__ float split16_scale(float amax, float *scale) 
   return __uint_as_float((268u - e) << 23);
 }
 
+// An element y = v * inv as its fp16 pair. lo of an infinity is 0, so that
+// the products are the f32 ones (inf - inf would make them NaN); NaN stays in
+// hi.
+static __device__ __forceinline__ void split16(float y, _Float16 &hi, _Float16 &lo) {
+  hi = (_Float16)y;
+  const float rest = y - (float)hi;
+  lo = (_Float16)(rest == rest ? rest : 0.0f);
+}
+
 // Converts the 32-element group held by a 32-lane half-wave (one value per
 // lane, hl = lane within the half-wave) into planes of layout D (kernels.h)
 // and the group's meta.
@@ -69,8 +78,8 @@ static __device__ __forceinline__ void quantize_group(float v, int hl, int g, in
   if constexpr (D == kPlanesSplit16) {
     ActMeta mm;
     const float y = v * split16_scale(amax, &mm.scale);
-    const _Float16 hi = (_Float16)y;
-    const _Float16 lo = (_Float16)(y - (float)hi);
+    _Float16 hi, lo;
+    split16(y, hi, lo);
     _Float16 *q = (_Float16 *)act_q;
     q[(((size_t)g * 2 + 0) * M + m) * 32 + split16_pos(hl)] = hi;
     q[(((size_t)g * 2 + 1) * M + m) * 32 + split16_pos(hl)] = lo;

@@ -991,10 +991,10 @@ __global__ __launch_bounds__(kEmitThreads) void splitk_resid_emit_kernel(GemvArg
     v8h hi, lo;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-      const float yq = v[i] * inv_s;
-      const _Float16 hv = (_Float16)yq;
+      _Float16 hv, lv;
+      split16(v[i] * inv_s, hv, lv);
       hi[split16_pos(i)] = hv;
-      lo[split16_pos(i)] = (_Float16)(yq - (float)hv);
+      lo[split16_pos(i)] = lv;
     }
     mm.corr = 0;
     if (act) {

@@ -94,3 +94,32 @@ def test_noalloc_accepts_the_same_calls(gh, gctx):
             gctx.sync()
             assert float((y - want).abs().max() / want.abs().max()) < 1e-6
         L.glacier_hip_int4_weight_destroy(w)
+
+
+@pytest.mark.parametrize("m", [3, 17, 40, 130])
+def test_split16_infinities_are_the_f32_product(gh, gctx, m):
+    """An f32 infinity times a weight is an infinity of their signs (NaN for
+    weight 0), infinities of two signs and NaN give NaN, other rows and the
+    row's finite columns are untouched by it."""
+    n, k = 48, 256
+    packed = gh.synth_int4(19, 1, n * k // 2)
+    s16 = gh.synth_scales_f16(19, 2, n * k // 32)
+    u = np.stack([packed & 15, packed >> 4], -1).reshape(n, k).astype(np.float64) - 7
+    w = u * np.repeat(s16.view(np.float16).astype(np.float64).reshape(n, k // 32), 32, 1)
+    x = np.random.default_rng(m).standard_normal((m, k)).astype(np.float32)
+    clean = _proj(gh, gctx, packed, s16, n, k, x, gh.ACT_F32)
+    bad = x.copy()
+    bad[0, 5] = np.inf
+    bad[m // 2, 37] = -np.inf
+    bad[m - 1, [70, 71, 200]] = [np.inf, np.inf, -np.inf]
+    bad[1, 9] = np.nan
+    got = _proj(gh, gctx, packed, s16, n, k, bad, gh.ACT_F32)
+    with np.errstate(invalid="ignore"):
+        want = (bad.astype(np.float64)[:, None, :] * w[None]).sum(-1)
+    rows = {0, 1, m // 2, m - 1}
+    for r in range(m):
+        if r not in rows:
+            assert np.array_equal(got[r], clean[r])
+        else:
+            assert not np.isfinite(want[r]).any()
+            assert np.array_equal(got[r], want[r].astype(np.float32), equal_nan=True), r
