@@ -87,9 +87,23 @@ static __device__ __forceinline__ void quantize_group(float v, int hl, int g, in
     if (hl == 0) meta[(size_t)g * M + m] = mm;
     return;
   }
-  const float scale = amax / 127.0f;
+  float scale = amax / 127.0f;
   const float inv_s = scale == 0.0f ? 0.0f : 1.0f / scale;
-  const float y = v * inv_s;
+  float y = v * inv_s;
+  if constexpr (D == kPlanesDigits) {
+    // Elements that are not finite (y is NaN there, also for an infinity,
+    // whose group's inv_s is 0): one infinity is the digit of its sign under
+    // an infinite scale, the f32 product with every weight; a NaN, or several
+    // infinities, whose products a digit sum cannot keep apart, make the row
+    // NaN.
+    const int half = threadIdx.x & 32;
+    const uint32_t odd = (uint32_t)(__ballot(y != y) >> half);
+    if (odd) {
+      const bool nan = (uint32_t)(__ballot(v != v) >> half) || (odd & (odd - 1));
+      scale = nan ? NAN : INFINITY;
+      y = y != y ? copysignf(1.0f, v) : 0.0f;
+    }
+  }
   float q0f = roundf(y);
   q0f = fminf(fmaxf(q0f, -127.0f), 127.0f);
   int qd[3] = {(int)q0f, 0, 0};

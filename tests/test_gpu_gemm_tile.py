@@ -123,3 +123,30 @@ def test_split16_infinities_are_the_f32_product(gh, gctx, m):
         else:
             assert not np.isfinite(want[r]).any()
             assert np.array_equal(got[r], want[r].astype(np.float32), equal_nan=True), r
+
+
+@pytest.mark.parametrize("m", [1, 2])
+def test_digit_infinities(gh, gctx, m):
+    """Up to 2 rows (three-digit planes): one infinity in a group is the f32
+    product too; several in a group, or a NaN, make the row NaN."""
+    n, k = 48, 256
+    packed = gh.synth_int4(23, 1, n * k // 2)
+    s16 = gh.synth_scales_f16(23, 2, n * k // 32)
+    u = np.stack([packed & 15, packed >> 4], -1).reshape(n, k).astype(np.float64) - 7
+    w = u * np.repeat(s16.view(np.float16).astype(np.float64).reshape(n, k // 32), 32, 1)
+    x = np.random.default_rng(m).standard_normal((m, k)).astype(np.float32)
+    clean = _proj(gh, gctx, packed, s16, n, k, x, gh.ACT_F32)
+    for at in ({37: np.inf}, {37: -np.inf}, {5: np.inf, 70: np.inf}, {5: np.inf, 200: -np.inf},
+               {9: np.nan}, {9: np.nan, 11: np.inf}, {64: np.inf, 95: np.inf}):
+        bad = x.copy()
+        for i, v in at.items():
+            bad[0, i] = v
+        got = _proj(gh, gctx, packed, s16, n, k, bad, gh.ACT_F32)
+        assert np.array_equal(got[1:], clean[1:])
+        groups = [i // 32 for i in at]
+        if len(set(groups)) < len(groups):
+            assert np.isnan(got[0]).all()
+        else:
+            with np.errstate(invalid="ignore"):
+                want = (bad[0].astype(np.float64) * w).sum(-1)
+            assert np.array_equal(got[0], want.astype(np.float32), equal_nan=True), at
