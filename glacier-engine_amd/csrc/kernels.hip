@@ -1552,8 +1552,12 @@ static __device__ __forceinline__ void attn_f32_item(const float *qrow, const fl
 // (scalar dots, 512-position chunks) -> 9.3; the compensated exponents cost 0.2 of
 // them and take the mean error against 64 bits from 1.77e-7 to 1.42e-7 (1.67e-7 with
 // attn_decode_kernel).
+// kQ8: planes, if any are emitted, are Q8. The other two layouts' conversions
+// cost every fp16 variant 4 to 7 registers, <64, 2, 8> its fifth wave a SIMD
+// (28 / 4 heads of 128, contexts up to 256, 1 to 31 lanes: 8.47 to 9.20 us
+// with all three, 8.25 to 8.95 without).
 // ---------------------------------------------------------------------------
-template <int HD, int NT, int NW, bool KV32>
+template <int HD, int NT, int NW, bool KV32, bool kQ8>
 __global__ __launch_bounds__(64 * NW) void attn_list_kernel(
     const float *q, const void *pool, const int32_t *page_table, int max_pages,
     const int32_t *lane_of_row, const int32_t *ctx_len, int M, int layer, int num_layers, int Hq,
@@ -1614,7 +1618,11 @@ __global__ __launch_bounds__(64 * NW) void attn_list_kernel(
       if (nch == 1) {
         const float v = KV32 ? O / L : O * (1.0f / L);
         out[((size_t)m * Hq + qh0 + g) * HD + d] = v;
-        emit_group(pd, v, t & 31, ((qh0 + g) * HD + d) >> 5, m, M);
+        if (pd.q) {
+          const int og = ((qh0 + g) * HD + d) >> 5;
+          if constexpr (kQ8) quantize_group<kPlanesQ8>(v, t & 31, og, m, M, pd.q, pd.meta);
+          else quantize_group_d(pd.D, v, t & 31, og, m, M, pd.q, pd.meta);
+        }
       } else {
         float *rec = rbase + g * hstride + (size_t)ch * RS;
         if (d == 0) {
@@ -1942,10 +1950,15 @@ static hipError_t launch_attention_list(const float *q, const void *kv_pool, boo
   // one workgroup per work item up to a cap; the rest loop over the list
   const long items = (long)nch * num_kv_heads * M;
   const unsigned grid = (unsigned)std::min<long>(items, kAttnMaxGrid);
-#define GK_LIST(HD, NT, NW, KV32)                                                             \
-  hipLaunchKernelGGL((attn_list_kernel<HD, NT, NW, KV32>), dim3(grid), dim3(64 * NW), 0, st, q, \
-                     kv_pool, page_table, max_pages, lane_of_row, ctx_len, M, layer,           \
+  const bool q8 = !emit.q || emit.D == kPlanesQ8;
+#define GK_LIST_Q(HD, NT, NW, KV32, Q)                                                      \
+  hipLaunchKernelGGL((attn_list_kernel<HD, NT, NW, KV32, Q>), dim3(grid), dim3(64 * NW), 0, \
+                     st, q, kv_pool, page_table, max_pages, lane_of_row, ctx_len, M, layer, \
                      num_layers, num_heads, num_kv_heads, nch, max_ctx, scratch, out, emit)
+#define GK_LIST(HD, NT, NW, KV32)                                                        \
+  do {                                                                                   \
+    if (q8) GK_LIST_Q(HD, NT, NW, KV32, true); else GK_LIST_Q(HD, NT, NW, KV32, false);  \
+  } while (0)
 #define GK_LIST_HD(NT, NW, KV32)                                   \
   do {                                                             \
     if (head_dim == 64) GK_LIST(64, NT, NW, KV32);                 \
@@ -1961,6 +1974,7 @@ static hipError_t launch_attention_list(const float *q, const void *kv_pool, boo
   }
 #undef GK_LIST_HD
 #undef GK_LIST
+#undef GK_LIST_Q
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || nch <= 1) return e;
   if (head_dim == 64)
