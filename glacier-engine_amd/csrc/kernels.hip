@@ -863,25 +863,28 @@ hipError_t launch_gather_rows(const float *table, const int32_t *ids, int M, int
 static constexpr int kMaxChunk = 512;
 static constexpr int kMaxRecords = 1024;  // chunk records one combine merges
 static constexpr int kMaxGroup = 8;
-static constexpr long kAttnMaxGrid = 4096;  // fp16 attention: workgroups per launch at most
-static constexpr int kF16MinChunk = 64;      // fewest positions per fp16-KV work item
+static constexpr long kAttnMaxGrid = 4096;  // work-list attention: workgroups per launch at most
+static constexpr int kListMinChunk = 64;    // fewest positions per work item of the list
 
 // Chunk length: short contexts stay one chunk (no combine launch); long ones
 // are split until (chunks x KV heads x rows) >= 2048 work items or chunks of
-// 64 positions, so a few long lanes still spread over the whole chip.
+// 64 positions, so a few long lanes still spread over the whole chip, as far
+// as the combine merges the records.
 int attention_chunk(int max_ctx, int num_kv_heads, int M) {
   int ch = kMaxChunk;
   if (max_ctx > 2 * kMaxChunk)
-    while (ch > 64 && ((max_ctx + ch - 1) / ch) * num_kv_heads * M < 2048) ch /= 2;
+    while (ch > 64 && ((max_ctx + ch - 1) / ch) * num_kv_heads * M < 2048 &&
+           (max_ctx + ch / 2 - 1) / (ch / 2) <= kMaxRecords)
+      ch /= 2;
   return ch;
 }
 
 size_t attention_scratch_floats(int max_rows, int num_heads, int num_kv_heads, int head_dim,
                                 int max_ctx) {
-  // fp16 KV: a chunk record per kF16MinChunk positions and (row, query head)
-  size_t most = (size_t)max_rows * num_heads * ((max_ctx + kF16MinChunk - 1) / kF16MinChunk) *
+  // the work list: a record per kListMinChunk positions and (row, query head)
+  size_t most = (size_t)max_rows * num_heads * ((max_ctx + kListMinChunk - 1) / kListMinChunk) *
                 (2 + head_dim);
-  // f32 KV: the largest chunk-record set the planner produces for any row count
+  // attn_decode_kernel: the largest chunk-record set for any row count
   for (int M = 1; M <= max_rows; ++M) {
     const int ch = attention_chunk(max_ctx, num_kv_heads, M);
     const size_t nch = (size_t)(max_ctx + ch - 1) / ch;

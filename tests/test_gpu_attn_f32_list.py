@@ -135,3 +135,10 @@ def test_pages_of_minus_infinite_scores_weigh_nothing(gh, gctx, hd, c):
         want = torch.softmax(sc, -1) @ v[live].double()
         err = float((got[h] - want).abs().max() / want.abs().max())
         assert err < 1e-6, (h, err)
+
+
+@pytest.mark.parametrize("ctx,lanes,Hkv", [(65537, 1, 2), (70000, 1, 2), (70000, 3, 1)])
+def test_contexts_past_the_work_list(gh, gctx, ctx, lanes, Hkv):
+    """Over 65536 positions of few KV heads (attn_decode_kernel, at most 1024
+    records of a row)."""
+    _run(gh, gctx, [ctx] + [37] * (lanes - 1), ctx, 2 * Hkv, Hkv, 64, 11)
