@@ -1096,13 +1096,12 @@ static bool gemm_direct_emit(const GemvArgs &a, const GemmShape &s) {
   return a.out_q && a.epi == EPI_SWIGLU && s.ks == 1;
 }
 
-// Whether the planes a launch emits overlap the planes it reads.
+// Whether the SwiGLU planes a launch emits overlap the planes it reads: a
+// finished tile would overwrite what the others still read.
 static bool emit_overlaps_input(const GemvArgs &a) {
   const size_t in_bytes = (size_t)(a.K / 32) * plane_group_bytes(a.D) * a.M;
-  const size_t out_bytes =
-      a.out_q ? (size_t)(a.N / (a.epi == EPI_SWIGLU ? 64 : 32)) * plane_group_bytes(a.out_D) * a.M : 0;
-  return a.out_q && (const int8_t *)a.out_q < a.act_q + in_bytes &&
-         a.act_q < (const int8_t *)a.out_q + out_bytes;
+  const size_t out_bytes = (size_t)(a.N / 64) * plane_group_bytes(a.out_D) * a.M;
+  return a.out_q < a.act_q + in_bytes && a.act_q < a.out_q + out_bytes;
 }
 
 bool gemm_emit_ok(const GemvArgs &a) {
@@ -1110,10 +1109,10 @@ bool gemm_emit_ok(const GemvArgs &a) {
   if (!a.out_q || !a.out_meta || (a.out_D != kPlanesQ8 && a.out_D != kPlanesSplit16) ||
       !gemm_plan(a, s)) return false;
   if (s.ks != 1 && s.ks != 2 && s.ks != 4 && s.ks != 8 && s.ks != 16) return false;
-  if (a.epi == EPI_SWIGLU && gemm_direct_emit(a, s) && !emit_overlaps_input(a))
-    return (a.N / 2) % 32 == 0;
+  if (a.epi == EPI_SWIGLU && ((a.N / 2) % 32 || emit_overlaps_input(a))) return false;
+  if (gemm_direct_emit(a, s)) return true;
   if (!a.splitk_ws || (size_t)s.ks * a.M * a.N > a.splitk_ws_floats) return false;
-  if (a.epi == EPI_SWIGLU) return (a.N / 2) % 32 == 0;
+  if (a.epi == EPI_SWIGLU) return true;
   if (a.epi == EPI_RESID)
     return a.emit_norm_w && a.resid && a.y && a.N % 32 == 0 && a.N <= 8 * kEmitThreads;
   return false;
@@ -1129,17 +1128,13 @@ hipError_t launch_gemm(const GemvArgs &a, hipStream_t st) {
   // counters cover the grid, the tile has at most 32 rows and kFoldSplits
   // splits (their partial sums are read at once), and the epilogue is the
   // tile's own: any but the residual plane emission (whole-row RMSNorm);
-  // without a K split any tile emits SwiGLU's planes itself (never when the
-  // emitted planes overlap the input planes: a finished tile would
-  // overwrite what the others still read)
-  const bool overlap = emit_overlaps_input(a);
+  // without a K split any tile emits SwiGLU's planes itself
   const bool fold = (a.splitk_counters && s.grid <= a.splitk_counter_count && s.mt <= 2 &&
-                     (!emit || (a.epi == EPI_SWIGLU && !overlap)) && (s.ks > 1 || emit) &&
+                     (!emit || a.epi == EPI_SWIGLU) && (s.ks > 1 || emit) &&
                      s.ks <= kFoldSplits) ||
-                    (emit && !overlap && gemm_direct_emit(a, s));
+                    gemm_direct_emit(a, s);
   float *part = s.ks > 1 || (emit && !fold) ? a.splitk_ws : nullptr;
-  // (an emission that cannot fold, e.g. into its own input planes, needs
-  // the partial sums in the workspace)
+  // (an emission that cannot fold needs the partial sums in the workspace)
   if ((s.ks > 1 || (emit && !fold)) &&
       (!a.splitk_ws || (size_t)s.ks * a.M * a.N > a.splitk_ws_floats))
     return hipErrorInvalidValue;

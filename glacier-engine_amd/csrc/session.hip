@@ -1164,16 +1164,13 @@ hipError_t enqueue_layers(glacier_hip_session *s, int rows, const RowPtrs &rp, h
       } else {
         // GEMM: down's planes from gate/up's own tiles (the last K split of
         // each, or every tile without a split) or its finishing pass, else
-        // the SwiGLU rows; into act_q when gate/up reads O's planes from
-        // act_q2 (so no finished tile overwrites planes another still
-        // reads), else into act_q2 up to the rows it holds (gate/up then
-        // reads act_q: the conversion kernel's planes), else into act_q by
-        // the finishing pass
+        // the SwiGLU rows; into the buffer gate/up does not read, so that no
+        // finished tile overwrites planes another still reads: act_q when its
+        // planes are in act_q2, else (the conversion kernel's, in act_q, for
+        // rows that act_q2 holds at down's width) act_q2
         gout.emit = gin.planes_q == s->act_q2 ? gk::PlanesDst{s->act_q, s->act_meta, Dd}
-                    : (uint32_t)rows <= s->planes2_rows
-                        ? gk::PlanesDst{s->act_q2, s->act_meta2, Dd}
-                        : gk::PlanesDst{s->act_q, s->act_meta, Dd};
-        if (!gout.emit.q || !gemm_emit_ok(s, L.gu, Dg, rows, gk::EPI_SWIGLU, gin, gout)) {
+                                              : gk::PlanesDst{s->act_q2, s->act_meta2, Dd};
+        if (!gemm_emit_ok(s, L.gu, Dg, rows, gk::EPI_SWIGLU, gin, gout)) {
           gout.emit = gk::PlanesDst{nullptr, nullptr, 1};
           gout.y = s->act;
         }
