@@ -142,17 +142,20 @@ static __device__ __forceinline__ uint32_t here(uint32_t v) {
   return v;
 }
 
-// kRB: 16-row weight blocks per wave (1 or 2; the workgroup covers 4 kRB);
-// BM: activation rows per workgroup (16 or 32). The K quads are split over
+// kRB: 16-row weight blocks per wave (kRowBlocks<D>; the workgroup covers
+// 4 kRB); BM: activation rows per workgroup (16 or 32). The K quads are split over
 // blockIdx.y (ks_count splits); with part set each split writes its partial
 // sums to part [ks_count][M][N] (no epilogue; a finishing kernel runs it),
 // unless fold: then the splits of a tile meet at p.splitk_counters and the
 // last to arrive runs the epilogue (the SwiGLU plane emission included).
 // Lane (c, n) of a 16 x 16 output tile (row block i, row tile mt) holds rows
 // 16 mt + 4 c + r of column n.
-template <int D, int kRB, int BM>
-__global__ __launch_bounds__(256, kRB == 2 ? 4 : 5) void gemm_kernel(
+template <int D>
+constexpr int kRowBlocks = D == kPlanesQ8 ? 1 : 2;
+template <int D, int BM>
+__global__ __launch_bounds__(256, kRowBlocks<D> == 2 ? 4 : 5) void gemm_kernel(
     GemvArgs p, int m_tiles, int ks_count, float *part, int fold) {
+  constexpr int kRB = kRowBlocks<D>;
   using S = ActStage<D, BM>;
   constexpr int MT = BM / 16;         // 16-row activation tiles per wave
   constexpr int kNBW = kWaves * kRB;  // weight row blocks per workgroup
@@ -849,11 +852,9 @@ __global__ __launch_bounds__(kTileThreads, 4) void gemm_tile_kernel(GemvArgs p, 
 // Split-K finish: y = the fixed-order sum over splits of part[s][m][n],
 // through the same epilogue as the one-split kernel. One thread per output
 // (m, n); the SwiGLU / RoPE partner n ^ 8 is summed by the same thread.
-// KS > 0: that many splits, every load issued before the first add; KS = 0:
-// ks_count splits in a loop.
+// Every load is issued before the first add.
 template <int KS>
-__global__ __launch_bounds__(256) void splitk_reduce_kernel(GemvArgs p, int ks_count,
-                                                            const float *part) {
+__global__ __launch_bounds__(256) void splitk_reduce_kernel(GemvArgs p, const float *part) {
   const size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;
   const size_t MN = (size_t)p.M * p.N;
   if (idx >= MN) return;
@@ -862,28 +863,17 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(GemvArgs p, int ks_c
   const bool paired = p.epi == EPI_SWIGLU || p.epi == EPI_QKV;
   // the partner of an unpaired output is itself (loaded, never used)
   const size_t pi = paired ? (size_t)m * p.N + (n ^ 8) : idx;
-  float tot, partner;
-  if constexpr (KS > 0) {
-    float tv[KS], pv[KS];
+  float tv[KS], pv[KS];
 #pragma unroll
-    for (int s = 0; s < KS; ++s) {
-      tv[s] = part[s * MN + idx];
-      pv[s] = part[s * MN + pi];
-    }
-    tot = tv[0];
-    partner = pv[0];
+  for (int s = 0; s < KS; ++s) {
+    tv[s] = part[s * MN + idx];
+    pv[s] = part[s * MN + pi];
+  }
+  float tot = tv[0], partner = pv[0];
 #pragma unroll
-    for (int s = 1; s < KS; ++s) {
-      tot += tv[s];
-      partner += pv[s];
-    }
-  } else {
-    tot = part[idx];
-    partner = part[pi];
-    for (int s = 1; s < ks_count; ++s) {
-      tot += part[s * MN + idx];
-      partner += part[s * MN + pi];
-    }
+  for (int s = 1; s < KS; ++s) {
+    tot += tv[s];
+    partner += pv[s];
   }
   if (!paired) partner = 0.0f;
   store_output(p, p.epi, nb, n_local, m, tot, partner, epi_load(p, p.epi, nb, n_local, m));
@@ -1036,7 +1026,7 @@ GemmShape plan_gemm(int N, int M, int K, int D, size_t ws_floats) {
     // of MFMA and scaling work): 1 row block per wave for Q8, 2 for split-16,
     // toward about 1024 workgroups (sweeps of the 7B shapes)
     bm = M <= 16 ? 16 : 32;
-    s.nt = D == kPlanesQ8 ? 4 : 8;
+    s.nt = kWaves * (D == kPlanesQ8 ? kRowBlocks<kPlanesQ8> : kRowBlocks<kPlanesSplit16>);
     target = 1024;
   } else {
     // prompt chunks: 128-row tiles, 64-row ones where they round M up to so
@@ -1068,25 +1058,13 @@ size_t gemm_splitk_floats(int N, int M, int K, int D) {
   return s.ks > 1 ? (size_t)s.ks * M * N : 0;
 }
 
-// The launch shape of these arguments (plan_gemm plus the tuning
-// overrides); false when they are invalid.
+// The launch shape of these arguments; false when they are invalid.
 static bool gemm_plan(const GemvArgs &a, GemmShape &s) {
   if (a.N % 16 || a.K % 128 || a.M < 1 || !a.act_q || !a.act_meta ||
       (a.D != kPlanesQ8 && a.D != kPlanesSplit16))
     return false;
   if (a.ss_out || a.arg_parts || a.x_in) return false;  // GEMV-only
   s = plan_gemm(a.N, a.M, a.K, a.D, a.splitk_ws ? a.splitk_ws_floats : 0);
-  if (s.mt <= 2 && (a.rb_override == 1 || a.rb_override == 2)) {  // tuning
-    s.nt = 4 * a.rb_override;
-    s.n_tiles = (a.N / 16 + s.nt - 1) / s.nt;
-    s.grid = s.m_tiles * s.n_tiles;
-  }
-  if (a.ksplit_override > 0) {  // tuning: K splits (needs the workspace)
-    if ((size_t)a.ksplit_override * a.M * a.N > (a.splitk_ws ? a.splitk_ws_floats : 0) &&
-        a.ksplit_override > 1)
-      return false;
-    s.ks = std::min(a.ksplit_override, a.K / 128);
-  }
   return true;
 }
 
@@ -1108,7 +1086,6 @@ bool gemm_emit_ok(const GemvArgs &a) {
   GemmShape s;
   if (!a.out_q || !a.out_meta || (a.out_D != kPlanesQ8 && a.out_D != kPlanesSplit16) ||
       !gemm_plan(a, s)) return false;
-  if (s.ks != 1 && s.ks != 2 && s.ks != 4 && s.ks != 8 && s.ks != 16) return false;
   if (a.epi == EPI_SWIGLU && ((a.N / 2) % 32 || emit_overlaps_input(a))) return false;
   if (gemm_direct_emit(a, s)) return true;
   if (!a.splitk_ws || (size_t)s.ks * a.M * a.N > a.splitk_ws_floats) return false;
@@ -1138,14 +1115,9 @@ hipError_t launch_gemm(const GemvArgs &a, hipStream_t st) {
   if ((s.ks > 1 || (emit && !fold)) &&
       (!a.splitk_ws || (size_t)s.ks * a.M * a.N > a.splitk_ws_floats))
     return hipErrorInvalidValue;
-#define GK_GEMM(DD, RB, BM)                                                                      \
-  hipLaunchKernelGGL((gemm_kernel<DD, RB, BM>), grid, block, 0, st, a, s.m_tiles, s.ks, part, \
+#define GK_GEMM(DD, BM)                                                                      \
+  hipLaunchKernelGGL((gemm_kernel<DD, BM>), grid, block, 0, st, a, s.m_tiles, s.ks, part, \
                      fold ? 1 : 0)
-#define GK_GEMM_BM(DD, RB) \
-  do {                       \
-    if (s.mt == 1) GK_GEMM(DD, RB, 16);                           \
-    else GK_GEMM(DD, RB, 32);                                     \
-  } while (0)
 #define GK_TILE(DD, BM)                                                                          \
   hipLaunchKernelGGL((gemm_tile_kernel<DD, BM>), grid, dim3(kTileThreads), 0, st, a, s.m_tiles,  \
                      s.n_tiles, s.ks, part, fold ? 1 : 0)
@@ -1156,12 +1128,11 @@ hipError_t launch_gemm(const GemvArgs &a, hipStream_t st) {
       if (s.mt == 4) GK_TILE(kPlanesSplit16, 64); else GK_TILE(kPlanesSplit16, 128);
     }
   } else if (a.D == kPlanesQ8) {
-    if (s.nt == 8) GK_GEMM_BM(kPlanesQ8, 2); else GK_GEMM_BM(kPlanesQ8, 1);
+    if (s.mt == 1) GK_GEMM(kPlanesQ8, 16); else GK_GEMM(kPlanesQ8, 32);
   } else {
-    if (s.nt == 8) GK_GEMM_BM(kPlanesSplit16, 2); else GK_GEMM_BM(kPlanesSplit16, 1);
+    if (s.mt == 1) GK_GEMM(kPlanesSplit16, 16); else GK_GEMM(kPlanesSplit16, 32);
   }
 #undef GK_TILE
-#undef GK_GEMM_BM
 #undef GK_GEMM
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || fold) return e;
@@ -1197,11 +1168,10 @@ hipError_t launch_gemm(const GemvArgs &a, hipStream_t st) {
   const dim3 rg((unsigned)((MN + 255) / 256));
   const float *pc = part;
   switch (s.ks) {
-    case 2: hipLaunchKernelGGL((splitk_reduce_kernel<2>), rg, dim3(256), 0, st, a, s.ks, pc); break;
-    case 4: hipLaunchKernelGGL((splitk_reduce_kernel<4>), rg, dim3(256), 0, st, a, s.ks, pc); break;
-    case 8: hipLaunchKernelGGL((splitk_reduce_kernel<8>), rg, dim3(256), 0, st, a, s.ks, pc); break;
-    case 16: hipLaunchKernelGGL((splitk_reduce_kernel<16>), rg, dim3(256), 0, st, a, s.ks, pc); break;
-    default: hipLaunchKernelGGL((splitk_reduce_kernel<0>), rg, dim3(256), 0, st, a, s.ks, pc); break;
+    case 2: hipLaunchKernelGGL((splitk_reduce_kernel<2>), rg, dim3(256), 0, st, a, pc); break;
+    case 4: hipLaunchKernelGGL((splitk_reduce_kernel<4>), rg, dim3(256), 0, st, a, pc); break;
+    case 8: hipLaunchKernelGGL((splitk_reduce_kernel<8>), rg, dim3(256), 0, st, a, pc); break;
+    default: hipLaunchKernelGGL((splitk_reduce_kernel<16>), rg, dim3(256), 0, st, a, pc); break;
   }
   return hipGetLastError();
 }

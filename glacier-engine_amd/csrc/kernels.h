@@ -90,9 +90,6 @@ struct GemvArgs {
   float *y;                 // EPI_PLAIN/RESID: [M][N]; SWIGLU: [M][N/2]
   const float *resid;       // EPI_RESID
   int epi;
-  int ksplit_override;      // force the K split (tuning); 0 = heuristic
-  int rb_override;          // row blocks per workgroup with ksplit_override
-                            // (GEMM: 2 or 4 forces the row blocks per wave)
   int ksplit;               // set by launch_gemv
   int ksplit_lds_off;       // set by launch_gemv: LDS offset of the SwiGLU plane buffer
   QkvArgs qkv;
@@ -183,19 +180,19 @@ constexpr int planes_layout(bool q8, int rows) {
 // and epilogues as launch_gemv without the GEMV-only stages (partial sums of
 // squares, fused argmax, input mode; planes only through the finishing pass,
 // gemm_emit_ok). Block tile 16*mt activation rows x nt weight row blocks (16
-// rows each), 4 waves; ks > 1 splits K over workgroups, which needs
-// splitk_ws (ks * M * N floats) and a second, fixed-order reduction kernel.
-// ksplit_override / rb_override force the splits / row blocks per wave
-// (tuning).
+// rows each), 4 waves up to 32 rows and 8 above; ks > 1 splits K over
+// workgroups, which needs splitk_ws (ks * M * N floats) and, where the splits
+// do not fold, a second, fixed-order reduction kernel.
 struct GemmShape {
   int mt, nt, m_tiles, n_tiles, grid, ks;
 };
 GemmShape plan_gemm(int N, int M, int K, int D, size_t ws_floats);
-// Workspace floats the GEMM would use for these sizes with no limit.
 // True when launch_gemm can emit planes for these arguments (out_q set):
-// SwiGLU outputs or residual rows of at most 4096 in whole 32-wide groups,
-// a K split of 1, 2, 4, 8 or 16 and a workspace for its partial sums.
+// SwiGLU outputs (not over the planes the launch reads) or residual rows of
+// at most 4096, in whole 32-wide groups, and a workspace for the partial sums
+// where a finishing pass emits them.
 bool gemm_emit_ok(const GemvArgs &a);
+// Workspace floats the GEMM would use for these sizes with no limit.
 size_t gemm_splitk_floats(int N, int M, int K, int D);
 hipError_t launch_gemm(const GemvArgs &a, hipStream_t st);
 

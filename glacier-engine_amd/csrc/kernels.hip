@@ -671,9 +671,6 @@ __global__ __launch_bounds__(LB) void gemv_kernel(GemvArgs a) {
   }
 }
 
-// 3..5 rows of one-digit planes that fit in LDS run the batched dot4 kernel
-// (its cost grows with every row; from 8 rows on the MFMA kernel measured
-// faster on the 7B shapes, about even at 5).
 // Launch shape for these arguments; also fills the fields launch_gemv
 // derives (ksplit, LDS offsets). False when the arguments are invalid.
 static bool gemv_shape(GemvArgs &a, GemvShape &p) {
@@ -713,17 +710,6 @@ static bool gemv_shape(GemvArgs &a, GemvShape &p) {
     p.grid = (a.N / 16 + p.rb - 1) / p.rb;
     p.lds_bytes = std::max(p.lds_a ? planes_bytes(a.K / 32, a.M, a.D) + a.M * 4 : 0,
                            p.waves * red0);
-  }
-  if (a.ksplit_override > 0) {
-    if (a.arg_parts) return false;
-    p.ksplit = a.ksplit_override;
-    p.rb = a.rb_override > 0 ? a.rb_override : std::max(1, 4 / p.ksplit);
-    p.waves = p.ksplit * p.rb;
-    if (p.waves > 16 || p.ksplit > a.K / 128) return false;
-    p.grid = (a.N / 16 + p.rb - 1) / p.rb;
-    p.lds_bytes = std::max(p.lds_a ? planes_bytes(a.K / 32, a.M, a.D) + a.M * 4 : 0,
-                           p.waves * red0);
-    if (emit_planes && p.rb % 4) return false;
   }
   // input mode: the planes are built in LDS, so they must fit there
   if (a.x_in && !p.lds_a) return false;
