@@ -137,6 +137,13 @@ static __device__ __forceinline__ float quad_xor1(float v) {
 static __device__ __forceinline__ float quad_xor2(float v) {
   return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x4E, 0xF, 0xF, false));
 }
+// (lane 7 - l of each 8 and lane 15 - l of each row of 16)
+static __device__ __forceinline__ float row_half_mirror(float v) {
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x141, 0xF, 0xF, false));
+}
+static __device__ __forceinline__ float row_mirror(float v) {
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x140, 0xF, 0xF, false));
+}
 static __device__ __forceinline__ int quad_xor1(int v) { return __builtin_amdgcn_mov_dpp(v, 0xB1, 0xF, 0xF, false); }
 static __device__ __forceinline__ int quad_xor2(int v) { return __builtin_amdgcn_mov_dpp(v, 0x4E, 0xF, 0xF, false); }
 // Sum over the 16 lanes of each row by rotations 8, 4, 2, 1: every lane

@@ -1625,6 +1625,155 @@ __global__ __launch_bounds__(64 * NW) void attn_list_kernel(
   }
 }
 
+// ---------------------------------------------------------------------------
+// f32-KV decode attention of short contexts (up to 8 passes of positions): a
+// workgroup of 8 waves per (query head, KV head, row), so a few lanes
+// already use as many CUs as there are query heads. HD / 8 threads share a
+// position, and every thread holds its 8 dims of K and V of all its NP
+// positions in registers: q, K and V are requested before the first is used,
+// one trip past the page walk. Scores are f32 dots whose last lane sums keep
+// what they round off, and weights take it and the score's own rounding as in
+// attn_f32_item (error against 64-bit sums no larger than the work list's).
+// The waves' (max, sum, output) states merge by log-sum-exp in LDS.
+// Bound by the launch, the page walk and those loads. 1 / 8 lanes: 14 / 2
+// heads of 64 at 64 positions 6.0 / 6.2 us with the work list (4.6 / 4.6 with
+// scalar dots through LDS) -> 4.1 / 3.8, at 256 9.5 / 9.6 (6.8 / 6.9) -> 4.6 /
+// 4.3; 28 / 4 heads of 128 at 256 15.1 / 15.4 (9.9 / 15.7) -> 6.0 / 6.2.
+// ---------------------------------------------------------------------------
+static constexpr int kHeadWaves = 8;
+
+template <int HD, int NP>
+__global__ __launch_bounds__(64 * kHeadWaves) void attn_head_kernel(
+    const float *q, const float *pool, const int32_t *page_table, int max_pages,
+    const int32_t *lane_of_row, const int32_t *ctx_len, int M, int layer, int num_layers, int G,
+    int Hkv, uint32_t by_hkv, int max_ctx, float *out, PlanesDst pd) {
+  constexpr int TPP = HD / 8;               // threads per position
+  constexpr int PPW = 64 / TPP;             // positions of a wave per pass
+  constexpr int PPP = PPW * kHeadWaves;     // positions of a pass
+  static_assert(PPP % 16 == 0, "a thread keeps its page slot from pass to pass");
+  const int t = threadIdx.x, l = t & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(t >> 6);
+  // pair p of row and KV head; its query heads' workgroups share p % 8 and
+  // with it the XCD (hardware places block b on XCD b % 8), whose L2 then
+  // serves all but the first of them
+  const uint32_t p = 8 * blockIdx.z + blockIdx.x;
+  const int m = Hkv == 1 ? (int)p : (int)__umulhi(p, by_hkv);  // p / Hkv
+  if (m >= M) return;
+  const int h = (int)p - m * Hkv, qh = h * G + (int)blockIdx.y;
+  const int Hq = G * Hkv, kv_dim = Hkv * HD;
+  const int sub = l % TPP, pp = PPW * wv + l / TPP;  // position pp + PPP * i
+  const float *qr = q + ((size_t)m * Hq + qh) * HD + 8 * sub;
+  const float4 q0 = *(const float4 *)qr, q1 = *(const float4 *)(qr + 4);
+  const int ctx = min(ctx_len[m], max_ctx), lane = lane_of_row[m];
+  __builtin_amdgcn_sched_barrier(0);  // (all of these before the branch)
+  if (ctx <= 0) return;
+  // (loads past the context read its last page: in range, masked by value)
+  const int32_t *pt = page_table + (size_t)lane * max_pages;
+  const size_t in_page = (size_t)(pp & 15) * kv_dim + (size_t)h * HD + 8 * sub;
+  float4 k[NP][2], v[NP][2];
+  const float *rows[NP];
+  int page[NP];
+#pragma unroll
+  for (int i = 0; i < NP; ++i) page[i] = pt[min(PPP * i + PPW * wv, ctx - 1) >> 4];
+  __builtin_amdgcn_sched_barrier(0);  // (one wait for all of them)
+#pragma unroll
+  for (int i = 0; i < NP; ++i)
+    rows[i] = pool + ((size_t)page[i] * num_layers + layer) * 32 * kv_dim + in_page;
+#pragma unroll
+  for (int i = 0; i < NP; ++i) {
+    k[i][0] = *(const float4 *)rows[i];
+    k[i][1] = *(const float4 *)(rows[i] + 4);
+  }
+#pragma unroll
+  for (int i = 0; i < NP; ++i) {
+    v[i][0] = *(const float4 *)(rows[i] + 16 * kv_dim);
+    v[i][1] = *(const float4 *)(rows[i] + 16 * kv_dim + 4);
+  }
+  __builtin_amdgcn_sched_barrier(0);  // (the scheduler would sink V's loads to their use)
+  const float scale = 1.0f / sqrtf((float)HD);
+  float sc[NP], tail[NP], mx = -INFINITY;
+#pragma unroll
+  for (int i = 0; i < NP; ++i) {
+    const float a = fmaf(q0.x, k[i][0].x, q0.y * k[i][0].y), b = fmaf(q0.z, k[i][0].z, q0.w * k[i][0].w);
+    const float c = fmaf(q1.x, k[i][1].x, q1.y * k[i][1].y), d = fmaf(q1.z, k[i][1].z, q1.w * k[i][1].w);
+    float s = (a + b) + (c + d), e;
+    s += quad_xor1(s);
+    if constexpr (TPP == 16) s += quad_xor2(s);
+    if constexpr (TPP == 8) {
+      s = two_sum(s, quad_xor2(s), e);
+    }
+    float r;
+    // lanes 7 - l of 8, then 15 - l of 16 (the halves are uniform by then)
+    if constexpr (TPP == 16) {
+      s = two_sum(s, row_half_mirror(s), e);
+      const float s2 = row_mirror(s), e2 = row_mirror(e);
+      s = two_sum(s, s2, r);
+      e = (e + e2) + r;
+    } else {
+      const float s2 = row_half_mirror(s), e2 = row_half_mirror(e);
+      s = two_sum(s, s2, r);
+      e = (e + e2) + r;
+    }
+    const float vs = s * scale;
+    tail[i] = fmaf(e, scale, fmaf(s, scale, -vs));
+    sc[i] = pp + PPP * i < ctx ? vs : -INFINITY;
+    mx = fmaxf(mx, sc[i]);
+  }
+  if constexpr (TPP == 8) mx = fmaxf(mx, row_xor8(mx));
+  mx = xor32_max(xor16_max(mx));
+  const float m0 = mx == -INFINITY ? 0.0f : mx;  // (no position here: weights of 0)
+  float sum = 0.0f, o[8];
+#pragma unroll
+  for (int d = 0; d < 8; ++d) o[d] = 0.0f;
+#pragma unroll
+  for (int i = 0; i < NP; ++i) {
+    float de;
+    const float r = two_sum(sc[i], -m0, de);
+    const float err = de + tail[i];
+    float w = expf(r);
+    if (fabsf(err) < 0x1p-8f) w = fmaf(w, err, w);
+    sum += w;
+    const bool in = pp + PPP * i < ctx;  // (a stale row may hold an infinity)
+    const float va[8] = {v[i][0].x, v[i][0].y, v[i][0].z, v[i][0].w,
+                         v[i][1].x, v[i][1].y, v[i][1].z, v[i][1].w};
+#pragma unroll
+    for (int d = 0; d < 8; ++d) o[d] = fmaf(w, in ? va[d] : 0.0f, o[d]);
+  }
+  if constexpr (TPP == 8) sum += row_xor8(sum);
+  sum = xor32_add(xor16_add(sum));
+#pragma unroll
+  for (int d = 0; d < 8; ++d) {
+    if constexpr (TPP == 8) o[d] += row_xor8(o[d]);
+    o[d] = xor32_add(xor16_add(o[d]));
+  }
+  __shared__ __align__(16) float so[kHeadWaves][HD];
+  __shared__ float sm[kHeadWaves], sl[kHeadWaves];
+  if (l < TPP) {
+    *(float4 *)&so[wv][8 * sub] = make_float4(o[0], o[1], o[2], o[3]);
+    *(float4 *)&so[wv][8 * sub + 4] = make_float4(o[4], o[5], o[6], o[7]);
+  }
+  if (l == 0) {
+    sm[wv] = mx;
+    sl[wv] = sum;
+  }
+  __syncthreads();
+  if (t >= HD) return;
+  float Mx = -INFINITY;
+#pragma unroll
+  for (int w = 0; w < kHeadWaves; ++w)
+    if (sl[w] > 0.0f) Mx = fmaxf(Mx, sm[w]);
+  float L = 0.0f, O = 0.0f;
+#pragma unroll
+  for (int w = 0; w < kHeadWaves; ++w) {
+    const float f = sl[w] > 0.0f ? expf(sm[w] - Mx) : 0.0f;
+    L = fmaf(sl[w], f, L);
+    O = fmaf(so[w][t], f, O);
+  }
+  const float y = O / L;
+  out[((size_t)m * Hq + qh) * HD + t] = y;
+  emit_group(pd, y, t & 31, (qh * HD + t) >> 5, m, M);
+}
+
 // Batch-1 decode: the attention of KV head h fused with h's K slice of the
 // O projection (AttnOArgs). Workgroup (bg, h) first requests its wave's O
 // weights (row block bg * NW + wave, the KQS quads of slice h) and its rows'
@@ -2345,6 +2494,36 @@ hipError_t launch_attention(const float *q, const void *kv_pool, int kv_f16,
   if (num_heads % num_kv_heads != 0 || num_heads / num_kv_heads > kMaxGroup)
     return hipErrorInvalidValue;
   if (head_dim != 64 && head_dim != 128) return hipErrorInvalidValue;
+  if (!kv_f16 && M >= 1 && M <= 64 && max_ctx >= 1) {
+    // short f32 contexts: passes of attn_head_kernel (64 positions each with
+    // heads of 64, 32 with 128) rounded up to 1, 2, 4 or 8, and as many
+    // workgroups as about two rounds of what the CUs hold (more passes, more
+    // registers); from there on sharing K and V between the query heads pays:
+    // 28 / 4 heads of 128, list against this at 64, 128, 256 positions: 16
+    // lanes 8.4 / 4.5, 10.4 / 5.8, 15.4 / 10.2 us, 64 lanes 8.8 / 9.3, 11.8 /
+    // 13.6, 21.0 / 34.5
+    const int need = (max_ctx * head_dim / 8 + 64 * kHeadWaves - 1) / (64 * kHeadWaves);
+    const int np = need <= 1 ? 1 : need <= 2 ? 2 : need <= 4 ? 4 : 8;
+    if (need <= 8 && M * num_heads <= std::min(1536, 4096 / np)) {
+      const dim3 grid(8, num_heads / num_kv_heads, (M * num_kv_heads + 7) / 8);
+      // ceil(2^32 / Hkv): exact for p < 2^13
+      const uint32_t by_hkv = (uint32_t)((0x100000000ull + num_kv_heads - 1) / num_kv_heads);
+#define GK_HEAD(HD, NP)                                                                        \
+  hipLaunchKernelGGL((attn_head_kernel<HD, NP>), grid, dim3(64 * kHeadWaves), 0, st, q,        \
+                     (const float *)kv_pool, page_table, max_pages, lane_of_row, ctx_len, M,   \
+                     layer, num_layers, num_heads / num_kv_heads, num_kv_heads, by_hkv, max_ctx, \
+                     out, emit)
+#define GK_HEAD_NP(HD)                                              \
+  do {                                                              \
+    if (np == 1) GK_HEAD(HD, 1); else if (np == 2) GK_HEAD(HD, 2);  \
+    else if (np == 4) GK_HEAD(HD, 4); else GK_HEAD(HD, 8);          \
+  } while (0)
+      if (head_dim == 64) GK_HEAD_NP(64); else GK_HEAD_NP(128);
+#undef GK_HEAD_NP
+#undef GK_HEAD
+      return hipGetLastError();
+    }
+  }
   // contexts up to 256 positions: one work item per (row, KV head), 8 waves x 2
   // pages of fp16 or 16 waves x 1 page of f32 (twice the registers a page),
   // no combine launch; longer ones: 64-position items of 4 waves x 1 page for

@@ -142,3 +142,29 @@ def test_contexts_past_the_work_list(gh, gctx, ctx, lanes, Hkv):
     """Over 65536 positions of few KV heads (attn_decode_kernel, at most 1024
     records of a row)."""
     _run(gh, gctx, [ctx] + [37] * (lanes - 1), ctx, 2 * Hkv, Hkv, 64, 11)
+
+
+@pytest.mark.parametrize("hd,max_ctx", [(64, c) for c in (63, 64, 65, 128, 129, 256, 257, 511, 512, 513)] +
+                         [(128, c) for c in (31, 32, 33, 64, 65, 128, 129, 255, 256, 257)])
+def test_passes_of_the_per_head_kernel(gh, gctx, hd, max_ctx):
+    """Contexts around a wave's positions and a pass, at max_ctx around 1, 2,
+    4 and 8 passes (heads of 64: 64 positions each, 128: 32) and past them."""
+    ctxs = [c for c in (1, 3, 4, 5, 8, 9, 16, 17, 31, 32, 33, 63, 64, 65, 100, 128, 200, 256, 300)
+            if c < max_ctx]
+    _run(gh, gctx, ctxs + [max_ctx], max_ctx, 6, 3, hd, max_ctx)
+
+
+@pytest.mark.parametrize("Hkv", [1, 3, 4, 7])
+@pytest.mark.parametrize("lanes", [1, 2, 7, 64])
+def test_pairs_over_the_xcds(gh, gctx, lanes, Hkv):
+    """Rows x KV heads that do and do not fill eights."""
+    _run(gh, gctx, [5 + i % 20 for i in range(lanes)], 24, 2 * Hkv, Hkv, 64, lanes)
+
+
+@pytest.mark.parametrize("hd,Hq,lanes,max_ctx", [
+    (64, 24, 64, 64), (64, 25, 64, 64), (64, 16, 64, 256), (64, 17, 64, 256), (64, 8, 64, 300),
+    (64, 9, 64, 300), (128, 24, 64, 64), (128, 16, 64, 128), (128, 17, 64, 128), (128, 8, 64, 256),
+    (128, 9, 64, 256)])
+def test_workgroups_around_the_line(gh, gctx, hd, Hq, lanes, max_ctx):
+    """Both sides of the workgroup count past which the work list runs."""
+    _run(gh, gctx, [1 + (37 * i) % max_ctx for i in range(lanes)], max_ctx, Hq, Hq, hd, Hq)
