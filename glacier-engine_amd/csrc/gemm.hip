@@ -135,6 +135,13 @@ static __device__ __forceinline__ float opaque(float v) {
   return v;
 }
 
+// First quad of K split s of ks (a power of two, at most 16). By a shift: as
+// 64-bit divisions the two bounds were 300 instructions in front of every
+// load: 16 x 9728 x 896 10.1 -> 9.7 us, 5 x 4608 x 3584 10.7 -> 10.2.
+static __device__ __forceinline__ int split_quad(uint32_t s, int KQ, int ks) {
+  return (int)(s * (uint32_t)KQ >> __builtin_ctz(ks));
+}
+
 // A lane offset the compiler may not widen outside the loop: loads then take a
 // scalar base and this one register (a 64-bit address pair per load otherwise).
 static __device__ __forceinline__ uint32_t here(uint32_t v) {
@@ -175,8 +182,8 @@ __global__ __launch_bounds__(256, kRowBlocks<D> == 2 ? 4 : 5) void gemm_kernel(
   const int m0 = m_tile * BM;
   const int nb0 = n_tile * kNBW + wave * kRB;  // this wave's first row block
   // this split's quads kq0 .. kq0 + nq - 1
-  const int kq0 = (int)(((long)blockIdx.y * KQ) / ks_count);
-  const int nq = (int)(((long)(blockIdx.y + 1) * KQ) / ks_count) - kq0;
+  const int kq0 = split_quad(blockIdx.y, KQ, ks_count);
+  const int nq = split_quad(blockIdx.y + 1, KQ, ks_count) - kq0;
   const auto row_of = [&](int mt, int r) {
     return m0 + 16 * mt + 4 * c + r;
   };
@@ -529,8 +536,8 @@ __global__ __launch_bounds__(kTileThreads, 4) void gemm_tile_kernel(GemvArgs p, 
   const int band_rows = min(kBand, m_tiles - kBand * band);
   const int n_tile = in_band / band_rows, m_tile = kBand * band + in_band % band_rows;
   const int m0 = m_tile * BM, nb_wg = n_tile * 8;
-  const int kq0 = (int)(((long)blockIdx.y * KQ) / ks_count);
-  const int nq = (int)(((long)(blockIdx.y + 1) * KQ) / ks_count) - kq0;
+  const int kq0 = split_quad(blockIdx.y, KQ, ks_count);
+  const int nq = split_quad(blockIdx.y + 1, KQ, ks_count) - kq0;
   const auto row_of = [&](int mt, int r) {
     return m0 + 32 * wm + (Q8 ? 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3) : 16 * mt + 4 * c + r);
   };
