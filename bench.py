@@ -57,12 +57,14 @@ def log(*a):
     print(*a, file=sys.stderr, flush=True)
 
 
-def gemv_bytes(n, k, m, digits=1):
-    """Algorithmic HBM bytes of one prepared GEMV launch: packed codes (K/2 per
-    row) + fp16 group scales (K/16 per row) + the activation planes it reads
-    (`digits` int8 bytes per element plus an 8-byte scale/correction per
-    32-element group, per row of M) + the f32 outputs."""
-    return n * k // 2 + n * k // 16 + m * k * digits + m * (k // 32) * 8 + m * n * 4
+def gemv_bytes(n, k, m, q8=True):
+    """Algorithmic HBM bytes of one prepared projection launch: packed codes
+    (K/2 per row) + fp16 group scales (K/16 per row) + the activation planes
+    it reads (per element 1 byte with Q8; with f32 activations 3 digits up to
+    2 rows, an fp16 pair of 4 bytes above; plus an 8-byte scale/correction
+    per 32-element group, per row of M) + the f32 outputs."""
+    elem = 1 if q8 else 3 if m <= 2 else 4
+    return n * k // 2 + n * k // 16 + m * k * elem + m * (k // 32) * 8 + m * n * 4
 
 
 MALL_BYTES = 256 << 20   # MI355X Infinity Cache; rotated weight copies must exceed it
@@ -91,7 +93,8 @@ def time_gemv(gh, ctx, torch, cw, m, reps, act, end_to_end_bf16=False):
     """Cold GEMV timing over the weight copies `cw`, HIP events on the launch
     stream around a captured graph. Prepared launches (activation planes made
     once, untimed: the decode chain produces them inside the previous kernel)
-    with Q8 or 3-digit f32 planes; or, with end_to_end_bf16, the whole
+    with Q8 or f32 planes (three digits up to 2 rows, an fp16 pair above); or,
+    with end_to_end_bf16, the whole
     glacier_hip_int4_gemv call on bf16 activations (the conversion launch
     included, BASELINE config 2's bf16 leg)."""
     L = gh.lib()
@@ -138,7 +141,7 @@ def time_gemv(gh, ctx, torch, cw, m, reps, act, end_to_end_bf16=False):
         b = n * k // 2 + n * k // 16 + m * k * 2 + m * n * 4
         mode = "bf16_in_" + ("q8" if act == gh.ACT_Q8 else "f32")
     else:
-        b = gemv_bytes(n, k, m, 1 if act == gh.ACT_Q8 else 3)
+        b = gemv_bytes(n, k, m, act == gh.ACT_Q8)
         mode = "q8" if act == gh.ACT_Q8 else "f32"
     return dict(N=n, K=k, M=m, act=mode, us=round(us, 2), bytes=b, gbs=round(b / us / 1e3, 1),
                 frac=round(b / us / 1e3 / HBM_PEAK_GBS, 4), weight_copies=copies)
@@ -183,7 +186,7 @@ def cpu_gemv(gh, ctx, torch, n, k, act):
             dt = time.perf_counter() - t0
             reps += 1
         res[th] = dt / (reps - 1)
-    b = gemv_bytes(n, k, 1, 1 if act == gh.ACT_Q8 else 3)
+    b = gemv_bytes(n, k, 1, act == gh.ACT_Q8)
     err = float(np.max(np.abs(got - want)) / np.max(np.abs(want)))
     return dict(threads=cores, us=round(res[cores] * 1e6, 1), gbs=round(b / res[cores] / 1e9, 2),
                 us_8_threads=round(res[8] * 1e6, 1), gbs_8_threads=round(b / res[8] / 1e9, 2),
