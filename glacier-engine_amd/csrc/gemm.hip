@@ -12,14 +12,16 @@
 //     -12582912 * ws) = RN(T * ws) (int4_ops.h), then one fma applies the
 //     activation scale into the running sum.
 //   * split-16: f32 activations as an fp16 pair per element (x / 2^e = hi + lo
-//     to 2^-23 of x), codes as exact halves, two fp16 MFMAs (one onto the
+//     to the larger of 2^-23 of x and 2^-39 of the group's largest), codes as
+//     exact halves, two fp16 MFMAs (one onto the
 //     other) per group with f32 accumulation, then the same two scales. Against
 //     three 7-bit digits on i8 MFMAs (three of them and five f32 / integer
 //     operations per output and group): 1999 x 3584 x 18944 1302 -> 840 us,
 //     error against 64-bit sums 5.9e-7 -> 4.7e-7.
 //
-// The per-group scaling (two f32 operations per output and group) bounds the
-// tall tiles by vector issue, not by the matrix cores. Two kernels:
+// The tall tiles' largest known cost is the vector work of the per-group
+// scaling (two f32 operations per output and group), not the matrix cores (see
+// there). Two kernels:
 //   * up to 32 rows, gemm_kernel: 4 waves over 16 or 32 rows, each wave its
 //     own weight row blocks. Each lane loads its own 16-byte tile slot per row
 //     block and quad (1 KB per wave, fully coalesced), two quads in flight;
@@ -467,13 +469,16 @@ __global__ __launch_bounds__(256, kRowBlocks<D> == 2 ? 4 : 5) void gemm_kernel(
 // Prompt chunks (more than 32 rows): BM x 128 output tiles by 8 waves, both
 // operands in LDS.
 //
-// Bound: vector issue. Per output and group two f32 operations (scale by ws,
-// then by as into the running sum) against one MFMA worth 1/128 of its time;
+// Cost: per output and group two f32 operations (scale by ws, then by as into
+// the running sum) against one MFMA worth 1/128 of its time;
 // MFMAs and vector work add up on this chip (a 32x32x32 i8 MFMA alone 35
 // cycles, 32 fmas alone 86, together 106), f32 operations issue at 2.4-2.9
 // cycles when at least two waves of a SIMD are ready and all operands are
 // plain vector registers (v_fma_mix_f32, conversions and scalar operands
-// 4.4-4.9), a single wave at 5-8. Hence:
+// 4.4-4.9), a single wave at 5-8. At those rates the instructions of the 2048
+// x 37888 x 3584 Q8 launch are 509 of its 740 us (counted: 4.0e8 VALU, 8.5e6
+// MFMAs over 1024 SIMDs at 2.4 GHz); what the other 30% is (the clock under
+// load, LDS reads, barriers) has not been measured. Hence:
 //   * the workgroup unpacks each quad's codes once (one 32-code slot, or one
 //     word, per thread) into LDS operands every wave reads, so unpacking
 //     costs 1/BM of an output instead of 1/(rows of a wave);
@@ -482,7 +487,8 @@ __global__ __launch_bounds__(256, kRowBlocks<D> == 2 ? 4 : 5) void gemm_kernel(
 //     leaves half the multipliers idle), split-16 on 16 x 16 x 32;
 //   * results are scaled by ws in one run and added in another (a dependent
 //     instruction right behind costs the double rate).
-// Stage: Q8 a quad, split-16 a group, double buffered, one barrier a stage.
+// Stage: Q8 a quad in two buffers, split-16 a group in three, one barrier a
+// stage.
 // ---------------------------------------------------------------------------
 constexpr int kTileThreads = 512;
 constexpr int kTileN = 128;  // columns: 8 row blocks
@@ -887,7 +893,7 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(GemvArgs p, const fl
 }
 
 // Split-K finish of the gate/up GEMM that also emits the down projection's
-// digit planes: one thread per SwiGLU output (m, o), o < N / 2, whose gate
+// planes: one thread per SwiGLU output (m, o), o < N / 2, whose gate
 // and up rows are device rows 16 (o / 8) + o % 8 and that + 8 (the
 // interleaved layout); every split sum in a fixed order, then the epilogue's
 // silu(g) * u. A half-wave holds 32 consecutive outputs of one row, which
@@ -920,7 +926,7 @@ __global__ __launch_bounds__(256) void splitk_swiglu_emit_kernel(GemvArgs p, con
 // Split-K finish of a residual GEMM (O, down) that also produces the next
 // projection's input: y = resid + (fixed-order sum of the splits) is
 // written, then the row's RMSNorm with emit_norm_w (kernels.zig:141-220:
-// y / sqrt(mean(y^2) + eps) * w) and the group quantiser give the digit
+// y / sqrt(mean(y^2) + eps) * w) and the group quantiser give the
 // planes prep_act_kernel would make from y. One workgroup per row; each
 // thread owns 8 consecutive outputs (two 16-byte loads per split, all of a
 // thread's loads issued before the first add), so 4 threads (one quad) hold

@@ -19,7 +19,9 @@
 //     T = sum_d 128^(D-1-d) * sum_k u_k * q_d[k]   (u = stored code).
 //   D = 2 (f32 as an fp16 pair, for the GEMM's fp16 MFMAs):
 //     q    fp16   [G][hi, lo][M][32], element k at split16_pos(k);
-//          hi + lo = x / 2^e to 2^-23 of x (2^e: a power of two per group)
+//          hi + lo = x / 2^e (2^e: a power of two per group) to 2^-23 of x, or
+//          to 2^-39 of the group's largest for elements below 2^-17 of it, whose
+//          lo is subnormal; an infinity is (inf, 0)
 //     meta {f32 scale = 2^(e + 10), 0} [G][M]
 #pragma once
 #include <hip/hip_runtime.h>
@@ -135,9 +137,10 @@ struct GemvArgs {
   // RMSNorm needs whole rows)
   unsigned *splitk_counters;
   int splitk_counter_count;
-  // GEMM with out_q set (launch_gemm, when gemm_emit_ok): the finishing
-  // pass also writes the next projection's planes (layout out_D). EPI_SWIGLU: the SwiGLU outputs (width N/2); EPI_RESID: y after
-  // the RMSNorm with these weights and in_eps (y itself is written too).
+  // GEMM with out_q set (launch_gemm, when gemm_emit_ok): the tiles or the
+  // finishing pass also write the next projection's planes (layout out_D).
+  // EPI_SWIGLU: the SwiGLU outputs (width N/2); EPI_RESID: y after the RMSNorm
+  // with these weights and in_eps (y itself is written too).
   const float *emit_norm_w;
 };
 
@@ -178,8 +181,7 @@ constexpr int planes_layout(bool q8, int rows) {
 
 // MFMA GEMM (K2) for more than kGemvMaxRows activation rows: same arguments
 // and epilogues as launch_gemv without the GEMV-only stages (partial sums of
-// squares, fused argmax, input mode; planes only through the finishing pass,
-// gemm_emit_ok). Block tile 16*mt activation rows x nt weight row blocks (16
+// squares, fused argmax, input mode; planes as gemm_emit_ok says). Block tile 16*mt activation rows x nt weight row blocks (16
 // rows each), 4 waves up to 32 rows and 8 above; ks > 1 splits K over
 // workgroups, which needs splitk_ws (ks * M * N floats) and, where the splits
 // do not fold, a second, fixed-order reduction kernel.

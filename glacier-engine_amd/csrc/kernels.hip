@@ -1058,32 +1058,8 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(
   }
 }
 
-// ---------------------------------------------------------------------------
-// Streaming decode attention (fp16 or f32 KV). The work list is every (row, KV head, chunk
-// of CH = NW * NT * 16 positions) with each row's chunks counted from its own
-// context length, rows in order; workgroup b takes items b, b + grid, ...,
-// so no chunk past a row's context is ever launched for it. A wave owns NT
-// pages of its chunk (16 positions each): it reads their page ids once
-// (wave-uniform scalar loads), issues every K and V load of them together
-// and keeps the softmax in registers:
-//   scores  S^T[pos][head] = K . Q^T on v_mfma_f32_16x16x16f16, q split into
-//           fp16 hi + lo so every product is exact in f32; lane (c, j) ends
-//           with head j's scores of positions 4c + r (r = 0..3) of a page,
-//   softmax max / exp / sum per head over the wave's positions (in-lane, then
-//           two cross-row shuffles),
-//   P.V     on v_mfma_f32_16x16x16f16 as well: the A operand is P[head j]
-//           [positions 4c .. 4c+3], which is exactly what lane (c, j) holds,
-//           split into fp16 hi + lo (V is exact in fp16, so the products
-//           are exact in f32); lane (c, j) supplies V[4c + r][DPL * j + e]
-//           for output block e from the DPL consecutive dims it read of each
-//           of its four V rows (one 16-byte load per row at hd 128), so V is
-//           read row-major and fully coalesced.
-// The waves' (max, sum, output) states merge by log-sum-exp in LDS. A row
-// whose context is one chunk writes its output normalised once by the sum
-// (forward.zig:515-528); otherwise every chunk writes a (max, sum, output)
-// record per query head for the combine kernel.
-// ---------------------------------------------------------------------------
-// LDS of one fp16 attention work item: every wave's (output, max, sum)
+// LDS of one work item of the streaming decode attention (attn_list_kernel and
+// attn_o_kernel below): every wave's (output, max, sum)
 // state and the log-sum-exp merge weights.
 template <int HD, int NW>
 struct AttnF16Lds {

@@ -798,8 +798,8 @@ int head_D(const glacier_hip_session *s, int rows) {
 }
 
 // One projection over `rows` activation rows with the given epilogue. The
-// input is an f32 matrix x (optionally RMS-normalised with norm_w) or int8
-// digit planes a producer already emitted. An f32 input is converted into
+// input is an f32 matrix x (optionally RMS-normalised with norm_w) or planes a
+// producer already emitted. An f32 input is converted into
 // planes (planes_layout: Q8, or f32 as digits or fp16 pairs) either by a separate
 // kernel or, for decode-sized row sets whose planes fit in LDS, by the GEMV
 // itself while its weights stream in; in that input mode the RMSNorm is

@@ -69,7 +69,10 @@ enum glacier_hip_dtype {
  *         32-element group s = max|x|/127, q = clamp(round(x/s), +-127), exact
  *         integer dot per group, f32 across groups.
  *  F32  — the reference's f32-activation path (int4_matmul.zig:215-311),
- *         computed to ~2^-22 relative accuracy (three 7-bit digit planes).
+ *         computed to ~2^-22 of each group's largest activation: three 7-bit
+ *         digit planes up to 2 rows, an fp16 hi + lo pair above. A product
+ *         with an infinity is the f32 one; up to 2 rows several infinities
+ *         in one 32-element group, or a NaN, make the row NaN.
  *  AUTO — the reference's x86 dispatch (int4_matmul.zig:372-374,461-463):
  *         F32 when out_f > 65536 or in_f > 16384, else Q8. */
 enum glacier_hip_activation {
@@ -321,7 +324,7 @@ int glacier_hip_int4_gemv_noalloc(glacier_hip_context *ctx, glacier_hip_int4_wei
 /* The same projection in two phases, as the reference splits it into
  * quantizeQ8Activation (int4_matmul.zig:537-560, glacier_q8_activation_quantize
  * int4_neon.c:453-486) and linearInt4WeightQ8Prepared (int4_matmul.zig:771):
- * the activation is converted once into device "digit planes" that several
+ * the activation is converted once into device planes that several
  * projections with the same in_f can share. activation must be Q8 or F32
  * (F32 = three 7-bit digit planes up to 2 rows, an fp16 hi + lo pair per
  * element above; planes belong to the m they were prepared for). act_dev must hold

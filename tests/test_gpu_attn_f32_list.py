@@ -1,7 +1,8 @@
 """f32-page decode attention through glacier_hip_paged_attention at the edges
-of its work list: 16-position pages, 64- and 256-position items, the line at
-max_ctx = 256, one and 64 lanes, group sizes 1 to 8, K / V beyond the fp16
-range, unused page slots holding NaN. Against 64-bit sums; bar 1e-6 of the
+of its kernels: 16-position pages, the per-head kernel's passes, the work
+list's 64- and 256-position items, the lines between them, one and 64 lanes,
+group sizes 1 to 8, K / V beyond the fp16 range, unused page slots holding
+NaN. Against 64-bit sums; bar 1e-6 of the
 largest output (f32 scores of |q . k| up to ~60: 2^-19 absolute before the
 1 / sqrt(hd) factor)."""
 import numpy as np
@@ -94,7 +95,7 @@ def _uniform(gh, gctx, q, k, v, hd):
 
 
 @pytest.mark.parametrize("size", [1.0, 3e4, 1e15])
-@pytest.mark.parametrize("c", [33, 300])
+@pytest.mark.parametrize("c", [33, 300, 600])
 @pytest.mark.parametrize("hd", [64, 128])
 def test_equal_scores_of_any_size_weigh_equally(gh, gctx, hd, c, size):
     """Equal K rows: the output is V's mean whatever their score is, also
@@ -113,7 +114,7 @@ def test_equal_scores_of_any_size_weigh_equally(gh, gctx, hd, c, size):
         assert err < 2e-6, (seed, err)
 
 
-@pytest.mark.parametrize("c", [64, 300])
+@pytest.mark.parametrize("c", [64, 300, 600])
 @pytest.mark.parametrize("hd", [64, 128])
 def test_pages_of_minus_infinite_scores_weigh_nothing(gh, gctx, hd, c):
     """Whole pages whose scores overflow to -inf beside finite ones."""

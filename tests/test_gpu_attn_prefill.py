@@ -1,7 +1,7 @@
 """Edges of the prompt-chunk attention kernel (glacier_hip_paged_attention_prefill)
 against 64-bit sums: chunks around its 16-row wave tiles and 32-key stages,
-every group size from 1 to 8 query heads per KV head (1 to 8 waves, row tiles
-filled up to 8), both head widths, chunks that start mid-page, scattered
+every group size from 1 to 8 query heads per KV head (one row tile, or as many
+as fill 4 or 8 waves), both head widths, chunks that start mid-page, scattered
 pages whose unused slots hold NaN, and one row that dominates its softmax.
 
 Bar: 2e-6 of the largest output. Scores carry f32 accumulation rounding

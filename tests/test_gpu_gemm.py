@@ -1,14 +1,13 @@
-"""GPU parity of the MFMA GEMM (K2: projections over more than 2 rows, and
-3-digit ones from 3 rows; 16-row tiles up to 16 rows, 32-row tiles up to 32
-with K split over workgroups, 64-row tiles above)
-against the CPU oracle, through the C ABI (glacier_hip_int4_gemv with
-m > 5), and of chunked prefill end to end.
+"""GPU parity of the MFMA GEMM (K2: projections over more than 2 rows; 16-row
+tiles up to 16 rows, 32-row tiles up to 32, 64- or 128-row tiles above, K split
+over workgroups where the grid is small) against the CPU oracle, through the C
+ABI (glacier_hip_int4_gemv with m > 5), and of chunked prefill end to end.
 
 Tolerances: as the decode GEMV. Q8: every per-group integer dot is exact and
 the group term RN(T * s_w) is the reference's; the activation scale is folded
 into the running sum with one fused multiply-add (one rounding fewer per
 group than the reference's separate multiply and add) and the across-group
-order differs -> 2e-6 of max|y|. F32 (three 7-bit digit planes) -> 1e-5.
+order differs -> 2e-6 of max|y|. F32 (fp16 hi + lo pairs) -> 1e-5.
 At the config sizes (M = 2048, the 7B prefill projections) a sample of the
 rows is checked directly against the oracle (linear_int4_q8 /
 linear_int4_f32), and the same rows recomputed as 16- and 24-row GEMMs must
