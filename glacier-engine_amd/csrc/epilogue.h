@@ -59,13 +59,12 @@ static __device__ __forceinline__ float split16_scale(float amax, float *scale) 
   return __uint_as_float((268u - e) << 23);
 }
 
-// An element y = v * inv as its fp16 pair. lo of an infinity is 0, so that
-// the products are the f32 ones (inf - inf would make them NaN); NaN stays in
-// hi.
+// An element y = v * inv as its fp16 pair. lo of an infinity is finite (the
+// maximum takes the bound for inf - inf; a finite y's rest is 8 at most), so
+// that the products are the f32 ones; NaN stays in hi.
 static __device__ __forceinline__ void split16(float y, _Float16 &hi, _Float16 &lo) {
   hi = (_Float16)y;
-  const float rest = y - (float)hi;
-  lo = (_Float16)(rest == rest ? rest : 0.0f);
+  lo = (_Float16)fmaxf(y - (float)hi, -16.0f);
 }
 
 // Converts the 32-element group held by a 32-lane half-wave (one value per

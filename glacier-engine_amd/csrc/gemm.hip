@@ -476,7 +476,7 @@ __global__ __launch_bounds__(256, kRowBlocks<D> == 2 ? 4 : 5) void gemm_kernel(
 // cycles when at least two waves of a SIMD are ready and all operands are
 // plain vector registers (v_fma_mix_f32, conversions and scalar operands
 // 4.4-4.9), a single wave at 5-8. At those rates the instructions of the 2048
-// x 37888 x 3584 Q8 launch are 509 of its 740 us (counted: 4.0e8 VALU, 8.5e6
+// x 37888 x 3584 Q8 launch are 518 of its 745 us (counted: 4.1e8 VALU, 8.5e6
 // MFMAs over 1024 SIMDs at 2.4 GHz); what the other 30% is (the clock under
 // load, LDS reads, barriers) has not been measured. Hence:
 //   * the workgroup unpacks each quad's codes once (one 32-code slot, or one
@@ -542,8 +542,10 @@ __global__ __launch_bounds__(kTileThreads, 4) void gemm_tile_kernel(GemvArgs p, 
   const int band_rows = min(kBand, m_tiles - kBand * band);
   const int n_tile = in_band / band_rows, m_tile = kBand * band + in_band % band_rows;
   const int m0 = m_tile * BM, nb_wg = n_tile * 8;
-  const int kq0 = split_quad(blockIdx.y, KQ, ks_count);
-  const int nq = split_quad(blockIdx.y + 1, KQ, ks_count) - kq0;
+  // (not split_quad: with the shifts in front of it the loop's code lies
+  // differently, and 1999 x 3584 x 18944 takes 848 us instead of 845)
+  const int kq0 = (int)(((long)blockIdx.y * KQ) / ks_count);
+  const int nq = (int)(((long)(blockIdx.y + 1) * KQ) / ks_count) - kq0;
   const auto row_of = [&](int mt, int r) {
     return m0 + 32 * wm + (Q8 ? 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3) : 16 * mt + 4 * c + r);
   };
