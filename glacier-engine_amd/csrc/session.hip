@@ -1148,7 +1148,7 @@ hipError_t enqueue_layers(glacier_hip_session *s, int rows, const RowPtrs &rp, h
       // (where O has no finishing pass and act_q2 holds no planes of down's
       // width for these rows, gate/up's own go there, which fits every row at
       // model width, so that its tiles may emit down's into act_q: a 7B
-      // prompt of 2048 tokens 57.9 -> 52.6 ms against converting f32 SwiGLU rows)
+      // prompt of 2048 tokens 59.8 -> 56.1 ms against converting f32 SwiGLU rows)
       const bool convert2 = !chain && !oout.emit.q && (uint32_t)rows > s->planes2_rows;
       if (oout.emit.q || convert2) {
         gin.planes_q = s->act_q2;
