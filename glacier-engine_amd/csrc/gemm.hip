@@ -1032,40 +1032,53 @@ __global__ __launch_bounds__(kEmitThreads) void splitk_resid_emit_kernel(GemvArg
 
 }  // namespace
 
-GemmShape plan_gemm(int N, int M, int K, int D, size_t ws_floats) {
+// Tiles of bm rows x nt row blocks, K split over workgroups (at least 2 quads
+// each) toward `target` of them, as far as the partial sums fit the workspace.
+static GemmShape tiles(int N, int M, int K, int bm, int nt, int target, size_t ws_floats) {
   GemmShape s;
   const int NB = N / 16, KQ = K / 128;
-  int bm, target;
-  if (M <= 32) {
-    // decode lanes (16 rows up to 16, so small batches do not pay for 32 rows
-    // of MFMA and scaling work): 1 row block per wave for Q8, 2 for split-16,
-    // toward about 1024 workgroups (sweeps of the 7B shapes)
-    bm = M <= 16 ? 16 : 32;
-    s.nt = kWaves * (D == kPlanesQ8 ? kRowBlocks<kPlanesQ8> : kRowBlocks<kPlanesSplit16>);
-    target = 1024;
-  } else {
-    // prompt chunks: 128-row tiles, 64-row ones where they round M up to so
-    // many fewer rows that they win (a row of theirs costs 1.2 of a 128-row
-    // tile's with Q8, 1.3 with split-16: 2048 x 18944 x 3584 454 against 390
-    // us, 1999 x 3584 x 18944 1050 against 845), toward one workgroup a CU
-    // (M = 100, 3584 x 18944: 65 us with 256, 66 with 1024; M = 200, 3584 x
-    // 3584 with 64-row tiles 25.5 against 28.4)
-    const long r64 = (M + 63) / 64 * 64, r128 = (M + 127) / 128 * 128;
-    bm = r64 * (D == kPlanesQ8 ? 12 : 13) < r128 * 10 ? 64 : 128;
-    s.nt = kTileN / 16;
-    target = 256;
-  }
+  s.nt = nt;
   s.mt = bm / 16;
   s.m_tiles = (M + bm - 1) / bm;
   s.n_tiles = (NB + s.nt - 1) / s.nt;
   s.grid = s.m_tiles * s.n_tiles;
-  // split K over workgroups (at least 2 quads each) toward the target, as far
-  // as the partial sums fit the workspace
   s.ks = 1;
   while (s.grid * s.ks < target && 2 * s.ks <= KQ / 2 && s.ks < 16 &&
          (size_t)(2 * s.ks) * M * N <= ws_floats)
     s.ks *= 2;
   return s;
+}
+
+// What a tile kernel's launch and its finishing pass take, in us to within the
+// choice this serves (fitted to both heights at 7 shapes of 40 to 2048 rows):
+// the most workgroups of a CU, two at a time (one alone takes 1.2 of its share
+// of two), times a workgroup's rows and quads (0.0103 us a row and quad with
+// Q8, 0.0184 with split-16, 1.3 times that in a 64-row tile); for a K split a
+// launch, its loads of ks partial sums and their bytes.
+static float tile_cost(const GemmShape &s, int N, int M, int K, int D) {
+  const int bm = 16 * s.mt, per_cu = (s.grid * s.ks + 255) / 256;
+  const float row = (D == kPlanesQ8 ? 0.0103f : 0.0184f) * (bm == 128 ? 1.0f : 1.3f);
+  const float run = (per_cu + 0.2f * (per_cu & 1)) * bm * row * (K / 128) / s.ks;
+  return s.ks == 1 ? run : run + 2.0f + 0.6f * s.ks + 0.5e-6f * s.ks * M * N;
+}
+
+GemmShape plan_gemm(int N, int M, int K, int D, size_t ws_floats) {
+  // decode lanes (16 rows up to 16, so small batches do not pay for 32 rows
+  // of MFMA and scaling work): 1 row block per wave for Q8, 2 for split-16,
+  // toward about 1024 workgroups (sweeps of the 7B shapes)
+  if (M <= 32)
+    return tiles(N, M, K, M <= 16 ? 16 : 32,
+                 kWaves * (D == kPlanesQ8 ? kRowBlocks<kPlanesQ8> : kRowBlocks<kPlanesSplit16>),
+                 1024, ws_floats);
+  // prompt chunks: 128- or 64-row tiles toward one workgroup a CU (M = 100,
+  // 3584 x 18944: 65 us with 256, 66 with 1024), whichever tile_cost finds
+  // cheaper: a row of a 64-row tile costs more, but they round M up to fewer
+  // rows, leave a fuller last round and split K less (us, 64 / 128 rows: 2048
+  // x 18944 x 3584 454 / 390, 554 x 3584 x 3584 43 / 53, 200 x 9728 x 896 19 /
+  // 28, 160 x 3584 x 18944 133 / 113)
+  const GemmShape s64 = tiles(N, M, K, 64, kTileN / 16, 256, ws_floats);
+  const GemmShape s128 = tiles(N, M, K, 128, kTileN / 16, 256, ws_floats);
+  return tile_cost(s64, N, M, K, D) < tile_cost(s128, N, M, K, D) ? s64 : s128;
 }
 
 size_t gemm_splitk_floats(int N, int M, int K, int D) {

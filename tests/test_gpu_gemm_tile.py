@@ -1,9 +1,9 @@
 """Edges of the prompt-chunk GEMM (gemm_tile_kernel) and of the split-16
 activation planes, through the C ABI against the CPU oracle and 64-bit sums.
 
-Rows around the 64- and 128-row tiles and the rule between them (64-row tiles
-at 33-64 and 129-192 rows), row blocks that do not fill a 128-column tile,
-K of one quad (one stage) and of K splits that divide unevenly. Bars as in
+Rows around the 64- and 128-row tiles, shapes that the rule between them gives
+to either, row blocks that do not fill a 128-column tile, K of one quad (one
+stage) and of K splits that divide unevenly. Bars as in
 test_gpu_gemm.py: Q8 2e-6 of max|y|, f32 1e-5.
 """
 import numpy as np
@@ -42,6 +42,31 @@ def test_tile_edges_match_oracle(gh, gctx, ora, n, k, m, act):
     fn = ora.linear_int4_q8 if act == "q8" else ora.linear_int4_f32
     want = fn(x, packed, s32, n, k, 32)
     err = np.max(np.abs(got - want)) / np.max(np.abs(want))
+    assert err < (2e-6 if act == "q8" else 1e-5), err
+
+
+@pytest.mark.parametrize("n,k,m", [(16400, 128, 193), (16400, 256, 255), (16400, 256, 257),
+                                   (16400, 640, 300), (16400, 384, 383), (4608, 3584, 250)])
+@pytest.mark.parametrize("act", ["q8", "f32"])
+def test_wide_outputs_match_64_bit_sums(gh, gctx, n, k, m, act):
+    """Enough columns for more than one 128-row tile a CU (the last shape with
+    a K split too); the same bars against 64-bit sums."""
+    import torch
+
+    packed = gh.synth_int4(n + k, 1, n * k // 2)
+    s16 = gh.synth_scales_f16(n + k, 2, n * k // 32)
+    x = np.random.default_rng(m).standard_normal((m, k)).astype(np.float32)
+    got = torch.from_numpy(_proj(gh, gctx, packed, s16, n, k, x,
+                                 gh.ACT_Q8 if act == "q8" else gh.ACT_F32)).cuda().double()
+    xv = x.reshape(m, -1, 32)
+    if act == "q8":  # group codes as the quantiser rounds them, half away from zero
+        sc = np.abs(xv).max(-1, keepdims=True) / np.float32(127)
+        r = xv * (np.float32(1) / sc)
+        xv = np.clip(np.sign(r) * np.floor(np.abs(r) + np.float32(0.5)), -127, 127) * sc.astype(np.float64)
+    u = torch.from_numpy(np.stack([packed & 15, packed >> 4], -1).reshape(n, k)).cuda()
+    w = (u.double() - 7).view(n, -1, 32) * torch.from_numpy(s16.view(np.float16).reshape(n, -1, 1)).cuda().double()
+    want = torch.from_numpy(xv.reshape(m, k).astype(np.float64)).cuda() @ w.view(n, k).t().contiguous()
+    err = float((got - want).abs().max() / want.abs().max())
     assert err < (2e-6 if act == "q8" else 1e-5), err
 
 
